@@ -1,0 +1,55 @@
+"""The token-tile kernels at the edges of their dispatch and of their tiles: 32-token tiles while one per CU
+covers the launch (256 CUs: 8,192 tokens), 64-token tiles beyond, partial last tiles, and for the per-op
+GEMMs widths that are not a multiple of a panel, of a k-step group or of the eight waves' tiles.
+
+References are the oracle's emulations of the same arithmetic, as in test_gpu_ops.py and test_gpu_blocks.py.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import folded, kernels as ok
+from turbo_roformer_amd import _hip, weights
+from turbo_roformer_amd.stack import HipStack
+
+from .conftest import assert_bf16_close, rand_x, snr_db
+
+DEV = "cuda"
+CFG = dict(weights.TINY_CFG, depth=1)
+
+
+def _weight(rows, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(rows, k, generator=g) / k**0.5).to(torch.bfloat16), torch.randn(rows, generator=g) * 0.1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [33, 8195])
+@pytest.mark.parametrize("K", [16, 144, 528, 1040])
+def test_gemm_res_norm_widths(hip, n, K):
+    W, b = _weight(256, K, K)
+    A = (rand_x(n, 60 + K).repeat(1, K // 256 + 1)[:, :K] * 0.5).to(torch.bfloat16).contiguous()
+    X = rand_x(n, 61, 2.0)
+    Xr, xnr = ok.gemm_res_norm(A, W, b, X)
+    Xd, xn = X.to(DEV), torch.empty(n, 256, dtype=torch.bfloat16, device=DEV)
+    print(f"gemm_res_norm K={K} n={n}", flush=True)
+    _hip.gemm_res_norm(A.to(DEV), _hip.pack_weight(W.to(DEV)), b.to(DEV), Xd, xn)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(Xd.cpu(), Xr, rtol=1e-5, atol=1e-5)  # fp32 sums of bf16 products
+    assert_bf16_close(xnr, xn, "xn", min_snr=55)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [33, 8195])
+@pytest.mark.parametrize("n_out", [32, 288, 544])
+def test_gemm_gelu_widths(hip, n, n_out):
+    W, b = _weight(n_out, 256, n_out)
+    xn = (rand_x(n, 70) * 0.5).to(torch.bfloat16)
+    Hr = ok.gemm_gelu(xn, W, b)
+    H = torch.empty(n, n_out, dtype=torch.bfloat16, device=DEV)
+    print(f"gemm_gelu n_out={n_out} n={n}", flush=True)
+    _hip.gemm_gelu(xn.to(DEV), _hip.pack_weight(W.to(DEV)), b.to(DEV), H)
+    torch.cuda.synchronize()
+    assert_bf16_close(Hr, H, "H", min_snr=50)

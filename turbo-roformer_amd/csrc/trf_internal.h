@@ -114,7 +114,7 @@ void launch_qkv_attn_short(const uint16_t* xn, const uint8_t* layer, const float
 // X += A [n][K] . W^T (+ bias), xn = X / max(|X|, eps) (W [256][K]); H = gelu_erf(xn . W^T + bias)
 // (W [n_out][256], n_out a multiple of 32).
 void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
-                          uint16_t* xn, int64_t n, float eps, hipStream_t st);
+                          uint16_t* xn, int64_t n, float eps, hipStream_t st, const LaunchEvents& ev = {});
 void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* bias, int n_out, uint16_t* H,
                       int64_t n, hipStream_t st);
 // Fused out-projection + residual + norm [+ FF1 + GELU + FF2 + residual + norm]; ff_precision is a

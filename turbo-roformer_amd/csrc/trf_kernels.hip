@@ -820,132 +820,7 @@ void launch_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* Vt, 
   }
 }
 
-// ============================================================ GEMM + residual + next norm
-// X[tok] += A[tok] . W^T (+ b); xn[tok] = X / max(|X|, eps), for any A width K (a multiple of 16) and a
-// weight W [256][K] packed in natural k order (launch_pack, kPack32Natural).  Each wave owns 32 tokens
-// and all 256 output features (8 accumulator tiles), so the row norm needs one half-wave swap.
-// (kernels.cpp:542-586)
-__global__ __launch_bounds__(256) void k_gemm_res_norm(const uint16_t* __restrict__ A, int K,
-                                                       const u32x4* __restrict__ wq, const float* __restrict__ bias,
-                                                       float* __restrict__ X, uint16_t* __restrict__ xn, int64_t n,
-                                                       float eps) {
-  const int KS = K / 16;
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int j = lane & 31, hh = lane >> 5;
-  const int64_t tok0 = (int64_t(blockIdx.x) * 4 + wave) * 32;
-  if (tok0 >= n) return;
-  const int64_t tok = tok0 + j;
-  const bool valid = tok < n;
-  const u32x4* ar = reinterpret_cast<const u32x4*>(A + (valid ? tok : 0) * K);
-
-  f32x16 acc[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = zero16();
-  for (int ks = 0; ks < KS; ++ks) {
-    const u32x4 b = valid ? ar[2 * ks + hh] : zero4();  // A[tok][16ks + 8hh .. +7]
-#pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = mfma32(wq[(int64_t(t) * KS + ks) * 64 + lane], b, acc[t]);
-  }
-  if (!valid) return;  // no cross-lane traffic below except the half-wave swap of valid pairs
-  float* xr = X + tok * kDim;
-  float ss = 0.f;
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int f0 = 32 * t + row_of_group(g, hh);
-      f32x4 x = *reinterpret_cast<const f32x4*>(xr + f0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float y = acc[t][4 * g + r] + x[r];
-        if (bias) y += bias[f0 + r];
-        acc[t][4 * g + r] = y;
-        x[r] = y;
-        ss = fmaf(y, y, ss);
-      }
-      *reinterpret_cast<f32x4*>(xr + f0) = x;
-    }
-  ss += __shfl_xor(ss, 32);
-  const float inv = 1.0f / fmaxf(sqrtf(ss), eps);
-  uint16_t* nr = xn + tok * kDim;
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int f0 = 32 * t + row_of_group(g, hh);
-      u32x2 v = {pk_bf16(acc[t][4 * g] * inv, acc[t][4 * g + 1] * inv),
-                 pk_bf16(acc[t][4 * g + 2] * inv, acc[t][4 * g + 3] * inv)};
-      *reinterpret_cast<u32x2*>(nr + f0) = v;
-    }
-}
-
-void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
-                          uint16_t* xn, int64_t n, float eps, hipStream_t st) {
-  hipLaunchKernelGGL(k_gemm_res_norm, dim3(unsigned((n + 127) / 128)), dim3(256), 0, st, A, K,
-                     reinterpret_cast<const u32x4*>(w_packed), bias, X, xn, n, eps);
-}
-
-// ============================================================ FF1 GEMM + GELU
-// H = 0.5 x (1 + erf(x / sqrt 2)), x = xn . W^T + b  (nn.GELU() default, model.py:69), for a weight
-// W [n_out][256] packed in natural k order (n_out a multiple of 32) and H [n][n_out].
-__global__ __launch_bounds__(256) void k_gemm_gelu(const uint16_t* __restrict__ xn, const u32x4* __restrict__ wq,
-                                                   const float* __restrict__ b1, int n_out,
-                                                   uint16_t* __restrict__ H, int64_t n) {
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int j = lane & 31, hh = lane >> 5;
-  const int64_t tok0 = (int64_t(blockIdx.x) * 4 + wave) * 32;
-  if (tok0 >= n) return;
-  const int64_t tok = tok0 + j;
-  const bool valid = tok < n;
-  const u32x4* xr = reinterpret_cast<const u32x4*>(xn + (valid ? tok : 0) * kDim);
-  u32x4 bx[16];
-#pragma unroll
-  for (int ks = 0; ks < 16; ++ks) bx[ks] = valid ? xr[2 * ks + hh] : zero4();  // natural k order
-  uint16_t* hr = H + (valid ? tok : 0) * int64_t(n_out);
-  for (int t = 0; t < n_out / 32; ++t) {
-    f32x16 acc = zero16();
-    const u32x4* w = wq + int64_t(t) * 16 * 64 + lane;
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks) acc = mfma32(w[ks * 64], bx[ks], acc);
-    if (valid) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int f0 = 32 * t + row_of_group(g, hh);
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float x = acc[4 * g + r] + b1[f0 + r];
-          v[r] = 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
-        }
-        u32x2 o = {pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3])};
-        *reinterpret_cast<u32x2*>(hr + f0) = o;
-      }
-    }
-  }
-}
-
-void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* bias, int n_out, uint16_t* H,
-                      int64_t n, hipStream_t st) {
-  hipLaunchKernelGGL(k_gemm_gelu, dim3(unsigned((n + 127) / 128)), dim3(256), 0, st, xn,
-                     reinterpret_cast<const u32x4*>(w_packed), bias, n_out, H, n);
-}
-
-// ============================================================ fused post-attention block
-// out-projection + residual + norm, then FF1 + GELU + FF2 + residual + norm, for 32 tokens per wave
-// (8 waves per workgroup, two per SIMD):
-//   acc  := O . Wout^T + X                     (8 stages of 4 k-steps; X joins one 32-row tile per stage)
-//   xn1  := acc / |acc|                        (FF1 B operands, in registers)
-//   for each of 32 hidden tiles u:  h = b1 + xn1 . W1t^T ; acc += gelu(h) . W2t^T
-//   acc  += b2 ; X := acc ; xn := acc / |acc|
-// xn1 and each GELU tile go from accumulator registers straight into B operands (W1, W2 are packed in
-// register order), so neither xn1 nor the 1024-wide hidden activation ever leaves the chip.
-// Replaces gemm_res_norm (out) + oneDNN FF1 + gemm_res_norm (FF2) (fast.py:311-331, kernels.cpp:542-642).
-constexpr int kMlpWaves = 8;
-constexpr int kOutStages = 8;                // 32 k-steps of W_out, 4 per stage
-constexpr int kFfStages = kHidden / 32;      // one 32-wide hidden tile per stage
-constexpr int kMlpPrefetch = 4;              // LDS operands read ahead of their MFMA (out-projection)
-constexpr int kMlpFfPrefetch = 2;            // the same in the feed-forward stages (registers are short)
-
+// ============================================================ GELU
 // erf-GELU x Phi(x) = max(x, 0) - 0.5|x| erfc(|x|/sqrt 2), with erfc from Abramowitz & Stegun 7.1.26
 // (|error of erf| <= 1.5e-7): erfc(z) = t (a1 + t (a2 + t (a3 + t (a4 + t a5)))) e^(-z^2),
 // t = 1/(1 + p z), p = 0.3275911.  Written in y = |x| sqrt(log2(e)/2) it is
@@ -993,6 +868,340 @@ __device__ __forceinline__ float gelu_logistic(float x) {
   const float e = __builtin_amdgcn_exp2f(-(x * p));
   return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
+
+// ============================================================ token-tile GEMM kernels
+// The kernels from here on give a workgroup a tile of 32 C tokens (C = 1 or 2) and all output features:
+// its 8 waves split the features (32-row weight tiles), and the tile's activations sit in LDS, where
+// every wave reads them as B operands.  A wave's weight tiles are its own, so they go from L2 straight
+// into registers as A operands, kWeightAhead k-steps ahead of their MFMAs: nothing waits at a barrier for
+// weights, and one 1 KB block feeds C MFMAs.  What C and the register budget are chosen for: two
+// workgroups of 8 waves per CU (at most 128 VGPRs and 80 KB of LDS each), so that one's memory phases and
+// barriers run beside the other's matrix work.  The L2 delivers ~50 bytes per cycle per CU, which bounds
+// C = 1 (1.3 MB of a sub-layer's weights per 32 tokens); C = 4 fills a CU with one workgroup.  Full
+// post-attention block, us at C = 1 / 2 / 4: 18 / 24 / 45 at 6,262 tokens, 37 / 35 / 53 at 16,384,
+// 223 / 172 / 225 at 105,462.  So a launch takes C = 1 while its 32-token tiles fit one per CU and
+// C = 2 beyond.
+//
+// Rows of X, O, xn and H move in whole rows or half rows per wave instruction and are transposed through
+// LDS.  Loaded or stored in operand layout (32 rows x 16 bytes, the halves of a pair 32 lanes apart) an
+// instruction occupies the CU's address path several times as long: the out-projection, residual and
+// norm alone took 89 us at 105,462 tokens that way, 72 us through LDS (378 MB: the HBM rate of a copy).
+// 1 KB rows are held as 64 16-byte chunks, chunk c of token t at c ^ (t & 15): the 16 lanes of an LDS
+// access then touch 16 different chunks of their 256 bytes.
+constexpr int kTileWaves = 8;
+constexpr int kWeightAhead = 4;  // k-steps a wave's weight blocks are loaded ahead (8 spills at C = 2)
+constexpr int kDropOffset = 0x7ffffff0;  // a buffer offset past every resource: its loads give zeros
+
+inline int token_tiles(int64_t n) { return n <= int64_t(32) * device_cu_count() ? 1 : 2; }
+
+__device__ __forceinline__ u32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+
+// This wave's LDS operations have completed, then all waves meet; its global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // vmcnt(63) expcnt(7) lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Everything this wave loads (direct-to-LDS loads too) has landed, then all waves meet.
+__device__ __forceinline__ void loads_barrier() {
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) expcnt(7) lgkmcnt(0)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Position of chunk c of token t in a tile of 1 KB rows.
+__device__ __forceinline__ int row_chunk(int t, int c) { return t * 64 + (c ^ (t & 15)); }
+
+// The norms of a tile's tokens: wave w's partial sum of squares of token t is ssq[t * kTileWaves + w].
+template <int C>
+__device__ __forceinline__ void put_ssq(const f32x16 (&acc)[C], float* ssq, int wave, int j, int hh) {
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct) {
+    float s = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s = fmaf(acc[ct][r], acc[ct][r], s);
+    s += __shfl_xor(s, 32);
+    if (hh == 0) ssq[(32 * ct + j) * kTileWaves + wave] = s;
+  }
+}
+
+__device__ __forceinline__ float inv_norm(const float* ssq, int t, float eps) {
+  const f32x4 p = *reinterpret_cast<const f32x4*>(ssq + t * kTileWaves);
+  const f32x4 q = *reinterpret_cast<const f32x4*>(ssq + t * kTileWaves + 4);
+  return 1.0f / fmaxf(sqrtf(((p[0] + p[1]) + (p[2] + p[3])) + ((q[0] + q[1]) + (q[2] + q[3]))), eps);
+}
+
+// The end of a tile: acc (tile `wave` of every token's features) -> X rows and, normalised, xn rows.
+// `rowbuf` holds the tile's fp32 rows; every wave has met since its last use, and since put_ssq.
+template <int C>
+__device__ __forceinline__ void store_tile(const f32x16 (&acc)[C], u32x4* rowbuf, const float* ssq, float eps,
+                                           __amdgpu_buffer_rsrc_t xres, __amdgpu_buffer_rsrc_t nres, int wave,
+                                           int lane) {
+  constexpr int RW = 32 * C / kTileWaves;
+  const int j = lane & 31, hh = lane >> 5;
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 x = {acc[ct][4 * g], acc[ct][4 * g + 1], acc[ct][4 * g + 2], acc[ct][4 * g + 3]};
+      rowbuf[row_chunk(32 * ct + j, 8 * wave + 2 * g + hh)] = __builtin_bit_cast(u32x4, x);
+    }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const int t = wave * RW + i;
+    const u32x4 v = rowbuf[row_chunk(t, lane)];
+    const f32x4 x = __builtin_bit_cast(f32x4, v);
+    const float inv = inv_norm(ssq, t, eps);
+    __builtin_amdgcn_raw_buffer_store_b128(v, xres, lane * 16 + t * (kDim * 4), 0, 0);
+    const u32x2 y = {pk_bf16(x[0] * inv, x[1] * inv), pk_bf16(x[2] * inv, x[3] * inv)};
+    __builtin_amdgcn_raw_buffer_store_b64(y, nres, lane * 8 + t * (kDim * 2), 0, 0);
+  }
+}
+
+// acc += x (or = x, INIT) for this wave's tile of features, from the tile's fp32 rows.
+template <int C, bool INIT>
+__device__ __forceinline__ void add_rows(const u32x4* rowbuf, f32x16 (&acc)[C], int wave, int j, int hh) {
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 x = __builtin_bit_cast(f32x4, rowbuf[row_chunk(32 * ct + j, 8 * wave + 2 * g + hh)]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[ct][4 * g + r] = INIT ? x[r] : acc[ct][4 * g + r] + x[r];
+    }
+}
+
+// ============================================================ GEMM + residual + next norm
+// X[tok] += A[tok] . W^T (+ b); xn[tok] = X / max(|X|, eps), for any A width K (a multiple of 16) and a
+// weight W [256][K] packed in natural k order (launch_pack, kPack32Natural); xn may be null (not written).
+// A is staged in panels of 512 columns (a row's chunks past K are dropped).  HBM-bound (378 MB at
+// 105,462 tokens and K = 512: 74 us at the rate of a copy; 486 MB and 95 us at K = 1024): 85 and 160 us, of
+// 269 and 512 for waves that read A and W from global memory as they multiplied, with no LDS.
+// (kernels.cpp:542-586)
+template <int C>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_res_norm(const uint16_t* __restrict__ A, int K,
+                                                                      const u32x4* __restrict__ wq,
+                                                                      const float* __restrict__ bias,
+                                                                      float* __restrict__ X,
+                                                                      uint16_t* __restrict__ xn, int64_t n,
+                                                                      float eps) {
+  constexpr int R = 32 * C, RW = R / kTileWaves;  // tokens of the tile, rows a wave moves
+  __shared__ u32x4 smem[R * 64 + R * kTileWaves / 4];
+  float* const ssq = reinterpret_cast<float*>(smem + R * 64);
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int j = lane & 31, hh = lane >> 5, t0 = wave * RW;
+  const int64_t tok0 = int64_t(blockIdx.x) * R;
+  const int rows = int(n - tok0 < R ? n - tok0 : R);
+  const auto xres = buffer_rsrc(X + tok0 * kDim, rows * kDim * 4);
+  const auto nres = buffer_rsrc(xn + tok0 * kDim, xn ? rows * kDim * 2 : 0);
+  const int KS = K / 16, chunks = K / 8, panels = (K + 511) / 512;
+  const auto wres = buffer_rsrc(wq + int64_t(wave) * KS * 64, KS * kTileBytes);
+  auto stage = [&](int panel) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const int t = t0 + i, c = 64 * panel + (lane ^ (t & 15));
+      const auto ares = buffer_rsrc(A + (tok0 + (t < rows ? t : 0)) * K, K * 2);  // one row
+      buffer_load_lds16(ares, c < chunks ? c * 16 : kDropOffset, smem + t * 64);
+    }
+  };
+  stage(0);
+  u32x4 xr[RW];
+#pragma unroll
+  for (int i = 0; i < RW; ++i) xr[i] = buffer_load16(xres, lane * 16 + (t0 + i) * (kDim * 4), 0);
+  auto weight = [&](int k) __attribute__((always_inline)) {  // k-step k (past the last one: the last, unused)
+    return buffer_load16(wres, lane * 16, min(k, KS - 1) * kTileBytes);
+  };
+  u32x4 a[kWeightAhead];
+#pragma unroll
+  for (int i = 0; i < kWeightAhead; ++i) a[i] = weight(i);
+  f32x16 acc[C];
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
+  const int m = j & 15, base = j * 64 + (hh ^ (m & 1)), me = m & 14;  // chunk 2k + hh of token j
+#pragma unroll 1
+  for (int panel = 0; panel < panels; ++panel) {
+    if (panel) {
+      lds_barrier();  // every wave has read the previous panel
+      stage(panel);
+    }
+    loads_barrier();
+    const int steps = min(32, KS - 32 * panel);
+#pragma unroll 1
+    for (int g = 0; g < steps / 8; ++g) {
+      const u32x4* p = smem + base + 16 * g;
+      const int next = 32 * panel + 8 * g + kWeightAhead;
+      u32x4 b[2][C];
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) b[0][ct] = p[me + ct * 32 * 64];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (k + 1 < 8) {
+#pragma unroll
+          for (int ct = 0; ct < C; ++ct) b[(k + 1) & 1][ct] = p[((2 * k + 2) ^ me) + ct * 32 * 64];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ct = 0; ct < C; ++ct) acc[ct] = mfma32(a[k % kWeightAhead], b[k & 1][ct], acc[ct]);
+        a[k % kWeightAhead] = weight(next + k);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll 1
+    for (int k = steps & ~7; k < steps; ++k) {  // K not a multiple of 128: only in the last panel
+      const u32x4 w = weight(32 * panel + k);
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma32(w, smem[base + ((2 * k) ^ me) + ct * 32 * 64], acc[ct]);
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < RW; ++i) smem[row_chunk(t0 + i, lane)] = xr[i];
+  lds_barrier();
+  add_rows<C, false>(smem, acc, wave, j, hh);
+  if (bias) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(bias + 32 * wave + row_of_group(g, hh));
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[ct][4 * g + r] += b[r];
+    }
+  }
+  put_ssq(acc, ssq, wave, j, hh);
+  lds_barrier();
+  store_tile(acc, smem, ssq, eps, xres, nres, wave, lane);
+}
+
+void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
+                          uint16_t* xn, int64_t n, float eps, hipStream_t st, const LaunchEvents& ev) {
+  const int C = token_tiles(n);
+  const auto kernel = C == 1 ? k_gemm_res_norm<1> : k_gemm_res_norm<2>;
+  hipExtLaunchKernelGGL(kernel, dim3(unsigned((n + 32 * C - 1) / (32 * C))), dim3(64 * kTileWaves), 0, st, ev.start,
+                        ev.stop, 0, A, K, reinterpret_cast<const u32x4*>(w_packed), bias, X, xn, n, eps);
+}
+
+// ============================================================ FF1 GEMM + GELU
+// H = 0.5 x (1 + erf(x / sqrt 2)), x = xn . W^T + b  (nn.GELU() default, model.py:69), for a weight
+// W [n_out][256] packed in natural k order (n_out a multiple of 32) and H [n][n_out].
+// 256 outputs (one weight tile per wave) at a time, through LDS into H as 16-byte chunks of whole rows:
+// position 32 t + (c ^ (t & 15)) for chunk c of token t, as for the tile's xn rows.
+// Bounded by the H writes (270 MB at 105,462 tokens, n_out = 1024: 53 us at the rate of a copy): 109 us, of
+// 267 for waves that read W from global memory one tile at a time and stored H in operand layout.
+template <int C>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_gelu(const uint16_t* __restrict__ xn,
+                                                                  const u32x4* __restrict__ wq,
+                                                                  const float* __restrict__ b1, int n_out,
+                                                                  uint16_t* __restrict__ H, int64_t n) {
+  constexpr int R = 32 * C;
+  __shared__ u32x4 smem[2 * R * 32];
+  u32x4* const hs = smem + R * 32;  // the outputs on their way out
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int j = lane & 31, hh = lane >> 5;
+  const int64_t tok0 = int64_t(blockIdx.x) * R;
+  const int rows = int(n - tok0 < R ? n - tok0 : R);
+  const auto nres = buffer_rsrc(xn + tok0 * kDim, rows * kDim * 2);
+  // 1 KB = two rows of 32 chunks per instruction; wave w moves instructions w, w + 8, ...
+  const int rp = lane >> 5, rc = lane & 31;
+#pragma unroll
+  for (int i = 0; i < R / 2 / kTileWaves; ++i) {
+    const int t = 2 * (kTileWaves * i + wave) + rp;
+    buffer_load_lds16(nres, t * (kDim * 2) + 16 * (rc ^ (t & 15)), smem + 2 * (kTileWaves * i + wave) * 32);
+  }
+  const int tiles = n_out / 32;
+  // weight tile t's blocks (past the last tile: the last one's, whose products are not stored)
+  auto tile_res = [&](int t) { return buffer_rsrc(wq + int64_t(min(t, tiles - 1)) * 16 * 64, 16 * kTileBytes); };
+  auto wr = tile_res(wave);
+  u32x4 a[kWeightAhead];
+#pragma unroll
+  for (int i = 0; i < kWeightAhead; ++i) a[i] = buffer_load16(wr, lane * 16, i * kTileBytes);
+  const int m = j & 15, base = j * 32 + (hh ^ (m & 1)), me = m & 14;  // chunk 2k + hh of token j
+  loads_barrier();
+#pragma unroll 1
+  for (int t8 = 0; t8 < tiles; t8 += kTileWaves) {
+    const int tile = t8 + wave;
+    const auto next = tile_res(tile + kTileWaves);
+    f32x16 acc[C];
+    {
+      f32x4 b[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        b[g] = *reinterpret_cast<const f32x4*>(b1 + (tile < tiles ? 32 * tile : 0) + row_of_group(g, hh));
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[ct][r] = b[r >> 2][r & 3];
+    }
+    u32x4 b[2][C];
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct) b[0][ct] = smem[base + me + ct * 32 * 32];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k + 1 < 16) {
+        const int c = ((2 * k + 2) & 16) + (((2 * k + 2) & 14) ^ me);
+#pragma unroll
+        for (int ct = 0; ct < C; ++ct) b[(k + 1) & 1][ct] = smem[base + c + ct * 32 * 32];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma32(a[k % kWeightAhead], b[k & 1][ct], acc[ct]);
+      if (k + kWeightAhead < 16)
+        a[k % kWeightAhead] = buffer_load16(wr, lane * 16, (k + kWeightAhead) * kTileBytes);
+      else
+        a[k % kWeightAhead] = buffer_load16(next, lane * 16, (k + kWeightAhead - 16) * kTileBytes);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    wr = next;
+    if (t8) lds_barrier();  // the previous 256 outputs have left hs
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {  // features 8g + 4hh .. +3 of this wave's tile: half hh of chunk 4 wave + g
+        const int t = 32 * ct + j;
+        const u32x2 v = {pk_bf16(gelu_erf(acc[ct][4 * g]), gelu_erf(acc[ct][4 * g + 1])),
+                         pk_bf16(gelu_erf(acc[ct][4 * g + 2]), gelu_erf(acc[ct][4 * g + 3]))};
+        reinterpret_cast<u32x2*>(hs)[2 * (t * 32 + ((4 * wave + g) ^ (t & 15))) + hh] = v;
+      }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < R / 2 / kTileWaves; ++i) {
+      const int t = 2 * (kTileWaves * i + wave) + rp;
+      const u32x4 v = hs[t * 32 + (rc ^ (t & 15))];
+      if (t < rows && 4 * t8 + rc < 4 * tiles)
+        *reinterpret_cast<u32x4*>(H + (tok0 + t) * n_out + 32 * t8 + 8 * rc) = v;
+    }
+  }
+}
+
+void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* bias, int n_out, uint16_t* H,
+                      int64_t n, hipStream_t st) {
+  const int C = token_tiles(n);
+  const auto kernel = C == 1 ? k_gemm_gelu<1> : k_gemm_gelu<2>;
+  hipLaunchKernelGGL(kernel, dim3(unsigned((n + 32 * C - 1) / (32 * C))), dim3(64 * kTileWaves), 0, st, xn,
+                     reinterpret_cast<const u32x4*>(w_packed), bias, n_out, H, n);
+}
+
+// ============================================================ fused post-attention block
+// out-projection + residual + norm, then FF1 + GELU + FF2 + residual + norm, for 32 tokens per wave
+// (8 waves per workgroup, two per SIMD):
+//   acc  := O . Wout^T + X                     (8 stages of 4 k-steps; X joins one 32-row tile per stage)
+//   xn1  := acc / |acc|                        (FF1 B operands, in registers)
+//   for each of 32 hidden tiles u:  h = b1 + xn1 . W1t^T ; acc += gelu(h) . W2t^T
+//   acc  += b2 ; X := acc ; xn := acc / |acc|
+// xn1 and each GELU tile go from accumulator registers straight into B operands (W1, W2 are packed in
+// register order), so neither xn1 nor the 1024-wide hidden activation ever leaves the chip.
+// Replaces gemm_res_norm (out) + oneDNN FF1 + gemm_res_norm (FF2) (fast.py:311-331, kernels.cpp:542-642).
+constexpr int kMlpWaves = 8;
+constexpr int kOutStages = 8;                // 32 k-steps of W_out, 4 per stage
+constexpr int kFfStages = kHidden / 32;      // one 32-wide hidden tile per stage
+constexpr int kMlpPrefetch = 4;              // LDS operands read ahead of their MFMA (out-projection)
+constexpr int kMlpFfPrefetch = 2;            // the same in the feed-forward stages (registers are short)
 
 __device__ __forceinline__ float acc_inv_norm(const f32x16 (&acc)[8], float eps) {
   float ss = 0.f;
