@@ -53,3 +53,47 @@ def test_gemm_gelu_widths(hip, n, n_out):
     _hip.gemm_gelu(xn.to(DEV), _hip.pack_weight(W.to(DEV)), b.to(DEV), H)
     torch.cuda.synchronize()
     assert_bf16_close(Hr, H, "H", min_snr=50)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["ff_fp16", "ff_split", "bf16"])
+@pytest.mark.parametrize("n", [1, 33, 8192, 8193])
+def test_feed_forward_tiles(hip, precision, n):
+    """The feed-forward sub-layer at both tile sizes; floors as in test_gpu_blocks.py."""
+    sd = weights.init_state_dict(CFG, seed=5, init="normal")
+    stack = HipStack(sd, DEV, precision=precision)
+    X = rand_x(n, 80 + n)
+    Xd = X.to(DEV)
+    print(f"feed-forward tiles n={n} {precision}", flush=True)
+    stack.ff_block(Xd, 1, n, 1, 0)
+    torch.cuda.synchronize()
+    P = folded.fold(sd, 1)[0]
+    if precision == "bf16":
+        w = ok.bf16_weights(P)
+        _, xn = ok.add_rmsnorm(X, None)
+        y, _ = ok.gemm_res_norm(ok.gemm_gelu(xn, w["W1"], w["b1"]), w["W2"], w["b2"], X)
+    else:
+        emulate = ok.ff_split if precision == "ff_split" else ok.ff_fp16
+        y, _ = emulate(X, P["W1"], P["b1"], P["W2"], P["b2"])
+    assert snr_db((y - X).numpy(), (Xd.cpu() - X).numpy()) >= 50.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["ff_fp16", "ff_split", "bf16"])
+@pytest.mark.parametrize("T,F", [(11, 3), (2765, 3)])
+def test_fused_block_matches_its_halves(hip, precision, T, F):
+    """Out-projection and feed-forward in one kernel (the stack) against the same as two (the attention
+    block's out-projection, then the feed-forward block).  They differ by the fp32 order of the residual
+    sums, which moves an operand of the feed-forward across a rounding boundary now and then: 60 dB allows
+    one half-step of bf16 (2^-9) in 1 of 4 operands."""
+    sd = weights.init_state_dict(CFG, seed=6, init="normal")
+    stack = HipStack(sd, DEV, precision=precision)
+    X = rand_x(T * F, 90).to(DEV)
+    print(f"fused block T={T} F={F} {precision}", flush=True)
+    got = stack(X.clone(), 1, T, F)
+    want = X.clone()
+    for layer in range(len(stack.modes)):
+        stack.attn_block(want, 1, T, F, layer)
+        stack.ff_block(want, 1, T, F, layer)
+    torch.cuda.synchronize()
+    assert snr_db((want - X).cpu().numpy(), (got - X).cpu().numpy()) >= 60.0

@@ -144,7 +144,11 @@ int run_layer(float* X, const trf::SeqShape& sh, const uint8_t* layer, const flo
     trf::launch_attention(w.Q, w.K, w.Vt, w.G, w.O, sh, st, ev.of(TRF_SLOT_ATTN));
     TRF_TRY(check_launch("attention"));
   }
-  trf::launch_post_attn(w.O, layer, X, w.xn, n, with_ff, ff_precision, 1e-12f, st, ev.of(TRF_SLOT_POST));
+  if (with_ff)
+    trf::launch_post_attn(w.O, layer, X, w.xn, n, ff_precision, 1e-12f, st, ev.of(TRF_SLOT_POST));
+  else  // nothing reads the workspace's xn after the block
+    trf::launch_gemm_res_norm(w.O, 512, layer + trf::kOffOut, nullptr, X, nullptr, n, 1e-12f, st,
+                              ev.of(TRF_SLOT_POST));
   return check_launch("post_attention");
 }
 
@@ -348,12 +352,9 @@ int trf_pack_layer(const trf_layer_src* src, void* dst, trf_stream_t stream) {
   trf::launch_copy_f32(src->b_ff1, trf::kHidden, reinterpret_cast<float*>(d + trf::kOffBff1), st);
   trf::launch_pack(src->w_ff2, trf::kDim, trf::kHidden, trf::kPack32RegOrder, d + trf::kOffFf2, st);
   trf::launch_copy_f32(src->b_ff2, trf::kDim, reinterpret_cast<float*>(d + trf::kOffBff2), st);
-  // operands of the split-bf16 feed-forward (16x16 tiles); absent lo parts pack as zeros
-  trf::launch_pack(src->w_out, trf::kDim, 512, trf::kPack16Natural, d + trf::kOffOut16, st);
-  trf::launch_pack(src->w_ff1, trf::kHidden, trf::kDim, trf::kPack16RegOrder, d + trf::kOffFf1Hi16, st);
-  trf::launch_pack(src->w_ff1_lo, trf::kHidden, trf::kDim, trf::kPack16RegOrder, d + trf::kOffFf1Lo16, st);
-  trf::launch_pack(src->w_ff2, trf::kDim, trf::kHidden, trf::kPack16RegOrder, d + trf::kOffFf2Hi16, st);
-  trf::launch_pack(src->w_ff2_lo, trf::kDim, trf::kHidden, trf::kPack16RegOrder, d + trf::kOffFf2Lo16, st);
+  // lo parts of the split-bf16 feed-forward; absent ones pack as zeros
+  trf::launch_pack(src->w_ff1_lo, trf::kHidden, trf::kDim, trf::kPack32RegOrder, d + trf::kOffFf1Lo, st);
+  trf::launch_pack(src->w_ff2_lo, trf::kDim, trf::kHidden, trf::kPack32RegOrder, d + trf::kOffFf2Lo, st);
   // operands of the fp16 feed-forward: fp16(hi + lo)
   trf::launch_pack_f16(src->w_ff1, src->w_ff1_lo, trf::kHidden, trf::kDim, d + trf::kOffFf1F16, st);
   trf::launch_pack_f16(src->w_ff2, src->w_ff2_lo, trf::kDim, trf::kHidden, d + trf::kOffFf2F16, st);
@@ -514,9 +515,7 @@ int trf_ff_block(float* X, int32_t batch, int32_t T, int32_t F, const void* pack
     return fail(TRF_ERR_WORKSPACE, "workspace is %zu bytes, need %zu", workspace_bytes, w.bytes);
   hipStream_t st = as_hip(stream);
   const int64_t n = int64_t(batch) * T * F;
-  trf::launch_add_rmsnorm(X, nullptr, 0, w.xn, 1, n, 1e-12f, st);
-  if (int rc = check_launch("add_rmsnorm")) return rc;
-  trf::launch_ff(static_cast<const uint8_t*>(packed_layer), X, w.xn, n, precision, 1e-12f, st);
+  trf::launch_ff(static_cast<const uint8_t*>(packed_layer), X, nullptr, n, precision, 1e-12f, st);
   return check_launch("feed_forward");
 }
 

@@ -35,18 +35,11 @@ constexpr size_t kOffBff1 = kOffFf1 + kSzFf1;
 constexpr size_t kOffFf2 = kOffBff1 + kHidden * 4;
 constexpr size_t kSzFf2 = size_t(kDim / 32) * (kHidden / 16) * kTileBytes;
 constexpr size_t kOffBff2 = kOffFf2 + kSzFf2;
-// The split-bf16 feed-forward runs on 16x16x32 MFMAs, whose A operand is 16 rows x 32 k: tiles
-// [rows/16][K/32][64 lanes][8 bf16], tile[t][ks][lane][e] = W[16t + lane%16][32ks + kperm16(lane/16, e)],
-// natural kperm16(g, e) = 8g + e (W_out), register order kperm16(g, e) = 16(e/4) + 4g + e%4 (W1, W2: a
-// 16x16 accumulator holds rows 4g..4g+3 in lane group g, so two tiles form one 32-deep B operand).
-// W1 and W2 come as hi = bf16(W) and lo = bf16(W - hi).
-constexpr size_t kOffOut16 = kOffBff2 + kDim * 4;
-constexpr size_t kOffFf1Hi16 = kOffOut16 + kSzOut;
-constexpr size_t kOffFf1Lo16 = kOffFf1Hi16 + kSzFf1;
-constexpr size_t kOffFf2Hi16 = kOffFf1Lo16 + kSzFf1;
-constexpr size_t kOffFf2Lo16 = kOffFf2Hi16 + kSzFf2;
+// The split-bf16 feed-forward takes W1 and W2 as hi = bf16(W) (the tiles above) and lo = bf16(W - hi).
+constexpr size_t kOffFf1Lo = kOffBff2 + kDim * 4;
+constexpr size_t kOffFf2Lo = kOffFf1Lo + kSzFf1;
 // fp16 W1 and W2 (32x32 register order, fp16(hi + lo)) for the fp16 feed-forward.
-constexpr size_t kOffFf1F16 = kOffFf2Lo16 + kSzFf2;
+constexpr size_t kOffFf1F16 = kOffFf2Lo + kSzFf2;
 constexpr size_t kOffFf2F16 = kOffFf1F16 + kSzFf1;
 constexpr size_t kLayerBytes = kOffFf2F16 + kSzFf2;
 
@@ -54,7 +47,7 @@ constexpr size_t kLayerBytes = kOffFf2F16 + kSzFf2;
 enum FfPrecision { kFfBf16 = 0, kFfSplit = 1, kFfFp16 = 2 };
 
 // Operand tile layouts of launch_pack.
-enum PackLayout { kPack32Natural = 0, kPack32RegOrder = 1, kPack16Natural = 2, kPack16RegOrder = 3 };
+enum PackLayout { kPack32Natural = 0, kPack32RegOrder = 1 };
 
 inline int32_t seq_pad(int32_t L) { return (L + 63) / 64 * 64; }
 
@@ -117,12 +110,13 @@ void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, con
                           uint16_t* xn, int64_t n, float eps, hipStream_t st, const LaunchEvents& ev = {});
 void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* bias, int n_out, uint16_t* H,
                       int64_t n, hipStream_t st);
-// Fused out-projection + residual + norm [+ FF1 + GELU + FF2 + residual + norm]; ff_precision is a
+// Fused out-projection + residual + norm + FF1 + GELU + FF2 + residual + norm; ff_precision is a
 // FfPrecision value for the two FF GEMMs.
-void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, bool with_ff,
-                      int ff_precision, float eps, hipStream_t st, const LaunchEvents& ev = {});
+void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision,
+                      float eps, hipStream_t st, const LaunchEvents& ev = {});
 // Fused FF1 + GELU + FF2 + residual + norm on X (updated in place, its norm computed in the kernel);
 // xn is written as X / |X|.
+// In these three xn may be null: it is then not written.
 void launch_ff(const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision, float eps, hipStream_t st);
 
 // ---------------------------------------------------------------- mask head (trf_mask.hip)

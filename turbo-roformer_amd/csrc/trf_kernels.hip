@@ -20,36 +20,26 @@
 namespace trf {
 
 // ============================================================ weight packing
-// 32x32 layouts: dst[t][ks][lane][e] = W[32t + lane%32][16ks + kperm(lane/32, e)] (kperm: natural 8hh + e,
-// or register order 4hh + e / 8 + 4hh + e - 4).  16x16 layouts: dst[t][ks][lane][e] =
-// W[16t + lane%16][32ks + kperm16(lane/16, e)] (natural 8g + e, register order 16(e/4) + 4g + e%4).
-// Rows past `rows` are zero, and so is everything when W is null.  (See trf_internal.h.)
+// dst[t][ks][lane][e] = W[32t + lane%32][16ks + kperm(lane/32, e)] (kperm: natural 8hh + e, or register order
+// 4hh + e / 8 + 4hh + e - 4).  Rows past `rows` are zero, and so is everything when W is null.  (See
+// trf_internal.h.)
 __global__ void k_pack(const uint16_t* __restrict__ W, int rows, int K, int layout, u32x4* __restrict__ dst) {
-  const bool t16 = layout >= kPack16Natural;
-  const int tr = t16 ? 16 : 32, kstep = t16 ? 32 : 16;
-  const int ksteps = K / kstep;
-  const int64_t total = int64_t((rows + tr - 1) / tr) * ksteps * 64;
+  const int ksteps = K / 16;
+  const int64_t total = int64_t((rows + 31) / 32) * ksteps * 64;
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= total) return;
   const int lane = int(i % 64);
   const int ks = int((i / 64) % ksteps);
   const int t = int(i / (64 * ksteps));
-  const int row = tr * t + lane % tr;
-  const int grp = lane / tr;
+  const int row = 32 * t + (lane & 31), hh = lane >> 5;
   u32x4 v = zero4();
   if (W && row < rows) {
-    const uint16_t* src = W + int64_t(row) * K + kstep * ks;
+    const uint16_t* src = W + int64_t(row) * K + 16 * ks;
     if (layout == kPack32Natural) {
-      v = *reinterpret_cast<const u32x4*>(src + 8 * grp);
-    } else if (layout == kPack32RegOrder) {
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src + 4 * grp);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8 + 4 * grp);
-      v = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    } else if (layout == kPack16Natural) {
-      v = *reinterpret_cast<const u32x4*>(src + 8 * grp);
+      v = *reinterpret_cast<const u32x4*>(src + 8 * hh);
     } else {
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(src + 4 * grp);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 16 + 4 * grp);
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(src + 4 * hh);
+      const u32x2 hi = *reinterpret_cast<const u32x2*>(src + 8 + 4 * hh);
       v = u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
   }
@@ -57,9 +47,7 @@ __global__ void k_pack(const uint16_t* __restrict__ W, int rows, int K, int layo
 }
 
 void launch_pack(const uint16_t* W, int rows, int K, int layout, uint8_t* dst, hipStream_t st) {
-  const bool t16 = layout >= kPack16Natural;
-  const int tr = t16 ? 16 : 32, kstep = t16 ? 32 : 16;
-  const int64_t total = int64_t((rows + tr - 1) / tr) * (K / kstep) * 64;
+  const int64_t total = int64_t((rows + 31) / 32) * (K / 16) * 64;
   hipLaunchKernelGGL(k_pack, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, W, rows, K, layout,
                      reinterpret_cast<u32x4*>(dst));
 }
@@ -1188,530 +1176,287 @@ void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* 
 }
 
 // ============================================================ fused post-attention block
-// out-projection + residual + norm, then FF1 + GELU + FF2 + residual + norm, for 32 tokens per wave
-// (8 waves per workgroup, two per SIMD):
-//   acc  := O . Wout^T + X                     (8 stages of 4 k-steps; X joins one 32-row tile per stage)
-//   xn1  := acc / |acc|                        (FF1 B operands, in registers)
-//   for each of 32 hidden tiles u:  h = b1 + xn1 . W1t^T ; acc += gelu(h) . W2t^T
+// out-projection + residual + norm, then FF1 + GELU + FF2 + residual + norm, for a tile of 32 C tokens:
+//   acc  := O . Wout^T + X                      (wave w: features 32w..32w+31 of every token)
+//   xn1  := acc / |acc|                         (FF1 B operands, in LDS)
+//   for each of 4 blocks c of 256 hidden units (wave w: units 256c + 32w ..+31):
+//     h   := b1 + xn1 . W1^T ;  gelu(h) -> LDS (FF2 B operands) ;  acc += gelu(h) . W2^T
 //   acc  += b2 ; X := acc ; xn := acc / |acc|
-// xn1 and each GELU tile go from accumulator registers straight into B operands (W1, W2 are packed in
-// register order), so neither xn1 nor the 1024-wide hidden activation ever leaves the chip.
-// Replaces gemm_res_norm (out) + oneDNN FF1 + gemm_res_norm (FF2) (fast.py:311-331, kernels.cpp:542-642).
-constexpr int kMlpWaves = 8;
-constexpr int kOutStages = 8;                // 32 k-steps of W_out, 4 per stage
-constexpr int kFfStages = kHidden / 32;      // one 32-wide hidden tile per stage
-constexpr int kMlpPrefetch = 4;              // LDS operands read ahead of their MFMA (out-projection)
-constexpr int kMlpFfPrefetch = 2;            // the same in the feed-forward stages (registers are short)
-
-__device__ __forceinline__ float acc_inv_norm(const f32x16 (&acc)[8], float eps) {
-  float ss = 0.f;
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) ss = fmaf(acc[t][r], acc[t][r], ss);
-  ss += __shfl_xor(ss, 32);
-  return 1.0f / fmaxf(sqrtf(ss), eps);
-}
-
-__device__ __forceinline__ void store_row(const f32x16 (&acc)[8], float inv, float* __restrict__ xr,
-                                          uint16_t* __restrict__ nr, int hh) {
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int f0 = 32 * t + row_of_group(g, hh);
-      f32x4 x = {acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
-      *reinterpret_cast<f32x4*>(xr + f0) = x;
-      u32x2 v = {pk_bf16(x[0] * inv, x[1] * inv), pk_bf16(x[2] * inv, x[3] * inv)};
-      *reinterpret_cast<u32x2*>(nr + f0) = v;
-    }
-}
-
-// FF1 / FF2 operand packing and product for the two feed-forward arithmetics of k_mlp.
-// F16: the two FF GEMMs take fp16 operands (xn, W1, gelu(h), W2; 11-bit significands instead of bf16's
-// 8) on v_mfma_f32_32x32x16_f16 with fp32 accumulation; the out-projection stays bf16.
-template <bool F16>
-__device__ __forceinline__ uint32_t pk_ff(float lo, float hi) {
-  return F16 ? pk_f16(lo, hi) : pk_bf16(lo, hi);
-}
-template <bool F16>
-__device__ __forceinline__ f32x16 mfma_ff(u32x4 a, u32x4 b, f32x16 c) {
-  return F16 ? mfma32h(a, b, c) : mfma32(a, b, c);
-}
-
-// This wave's 4 of stage s's 32 operand blocks into LDS.  Stages 0..7: W_out k-steps 4s..4s+3 of the
-// 8 tiles.  Feed-forward stage u = s - 8 (0..32): blocks 0..15 are W1 tile u (k-steps 0..15; none for
-// u = 32), blocks 16..31 W2 k-steps 2(u-1), 2(u-1)+1 of the 8 output tiles (for u = 0 k-steps 0, 1,
-// loaded but not read).  Nothing for s past the last stage.
-__device__ __forceinline__ void mlp_issue(int s, u32x4* dst, const u32x4* wo, const u32x4* w1, const u32x4* w2,
-                                          int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int b = wave * 4 + i;
-    const u32x4* src;
-    if (s < kOutStages) {
-      src = wo + (int64_t(b >> 2) * 32 + 4 * s + (b & 3)) * 64;  // W_out tile b/4, k-step 4s + b%4
-    } else {
-      const int u = s - kOutStages;
-      if (b < 16) {
-        if (u >= kFfStages) continue;
-        src = w1 + (int64_t(u) * 16 + b) * 64;  // W1 tile u, k-step b
-      } else {
-        if (u > kFfStages) continue;
-        src = w2 + (int64_t((b - 16) >> 1) * 64 + 2 * (u > 0 ? u - 1 : 0) + (b & 1)) * 64;  // W2 tile (b-16)/2
-      }
-    }
-    lds_load_block(src, dst + b * 64, lane);
-  }
-}
-
-// One feed-forward stage u, the same in every wave.  Stage u's LDS buffer holds W1 of hidden tile u
-// (blocks 0..15, k-steps 0..15) and W2 of tile u-1 (block 16 + 2t + c: output tile t, hidden half c).
-//   MFMAs 0..15:   FF1(u)   h := b1(u) + xn . W1(u)^T, one accumulator chain;
-//   MFMAs 16..31:  FF2(u-1) acc[t] += gelu(h(u-1))[half c] . W2(u-1, t, c)^T, step j = 16 + 8c + t.
-// GELU of the previous stage's h is spread between these MFMAs, value v after MFMA 3v/2, so that
-// neither wave of a SIMD runs a long VALU-only stretch: on gfx950 VALU work of one wave overlaps the
-// MFMAs of the other wave on its SIMD (measured: 65-80% of it hidden), while VALU work between a wave's
-// own MFMAs is barely hidden at all.  Values 0..7 (the B operand of steps 16..23) are done by MFMA 10,
-// values 8..15 by MFMA 22.
-// KIND 0: the first stage (FF1(0) only); KIND 1: stages 1..31; KIND 2: the last stage (FF2(31) only).
-constexpr int mlp_gelu_slot(int v) { return (3 * v) / 2; }
-
-__device__ __forceinline__ constexpr int mlp_block_of(int m) {
-  return m < 16 ? m : 16 + 2 * ((m - 16) % 8) + (m - 16) / 8;
-}
-
-template <bool F16, int KIND>
-__device__ __forceinline__ void mlp_ff_pstage(const u32x4* Ls, const f32x4* b1s, const u32x4 (&xb)[16], int u,
-                                              int hh, int lane, f32x16& h, f32x16 (&acc)[8]) {
-  constexpr int D = kMlpFfPrefetch;
-  constexpr int m0 = KIND == 2 ? 16 : 0, m1 = KIND == 0 ? 16 : 32;
-  const f32x16 hp = h;  // h(u-1), the GELU input (KIND 1, 2)
-  if (KIND != 2) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 b = b1s[8 * u + 2 * g + hh];  // h starts at b1
-#pragma unroll
-      for (int r = 0; r < 4; ++r) h[4 * g + r] = b[r];
-    }
-  }
-  u32x4 hb[2] = {zero4(), zero4()};
-  float gv[2];
-  auto gelu_value = [&](int v) {
-    gv[v & 1] = gelu_logistic(hp[v]);
-    if (v & 1) hb[v >> 3][(v & 7) >> 1] = pk_ff<F16>(gv[0], gv[1]);
-  };
-  if (KIND == 2) {  // nothing to hide the first half behind
-#pragma unroll
-    for (int v = 0; v < 8; ++v) gelu_value(v);
-  }
-  u32x4 a[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i)
-    if (m0 + i < m1) a[i] = Ls[mlp_block_of(m0 + i) * 64 + lane];
-#pragma unroll
-  for (int m = m0; m < m1; ++m) {
-    const int i = m - m0;
-    if (m < 16) {
-      h = mfma_ff<F16>(a[i % D], xb[m], h);
-    } else {
-      const int j = m - 16;
-      acc[j % 8] = mfma_ff<F16>(a[i % D], hb[j / 8], acc[j % 8]);
-    }
-    if (m + D < m1) a[i % D] = Ls[mlp_block_of(m + D) * 64 + lane];
-    if (KIND == 1) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if (mlp_gelu_slot(v) == m) gelu_value(v);
-    } else if (KIND == 2) {
-      if (m < 24) gelu_value(8 + (m - 16));  // values 8..15 beside steps 16..23 (half 0)
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// 32 out-projection MFMAs of one stage: MFMA i -> output tile i%8, k-step i/8 of the stage (block
-// 4(i%8) + i/8), operands read from LDS kMlpPrefetch ahead.
-__device__ __forceinline__ void mlp_out_block(const u32x4* Ls, const u32x4 (&cur)[4], int lane, f32x16 (&acc)[8]) {
-  constexpr int D = kMlpPrefetch;
-  u32x4 a[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) a[i] = Ls[(4 * (i % 8) + i / 8) * 64 + lane];
-#pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    acc[i % 8] = mfma32(a[i % D], cur[i / 8], acc[i % 8]);
-    if (i + D < 32) a[i % D] = Ls[(4 * ((i + D) % 8) + (i + D) / 8) * 64 + lane];
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// The 33 feed-forward stages.  Every wave runs the same sequence; before stage u all waves meet (stage
-// u's operands have landed and stage u-1's buffer is free) and stage u+1's operands are issued into
-// that buffer.  Stages go in pairs so that each one's buffers are compile-time constants: the compiler
-// can then tell the operand reads from the direct-to-LDS loads into the other buffer, and does not wait
-// for those loads before reading.
-template <bool F16>
-__device__ __forceinline__ void mlp_ff_stages(f32x16 (&acc)[8], const u32x4 (&xb)[16], u32x4 (*lds)[32 * 64],
-                                              const f32x4* b1s, const u32x4* wo, const u32x4* w1,
-                                              const u32x4* w2, int wave, int lane, int hh) {
-  constexpr int s0 = kOutStages;
-  static_assert(s0 % 2 == 0 && kFfStages == 32, "stage 0 in buffer 0, stages 1..30 in pairs");
-  f32x16 h = zero16();
-  stage_barrier();
-  mlp_issue(s0 + 1, lds[1], wo, w1, w2, wave, lane);
-  mlp_ff_pstage<F16, 0>(lds[0], b1s, xb, 0, hh, lane, h, acc);
-#pragma clang loop unroll(disable)
-  for (int u = 1; u < kFfStages - 1; u += 2) {
-    stage_barrier();
-    mlp_issue(s0 + u + 1, lds[0], wo, w1, w2, wave, lane);
-    mlp_ff_pstage<F16, 1>(lds[1], b1s, xb, u, hh, lane, h, acc);
-    stage_barrier();
-    mlp_issue(s0 + u + 2, lds[1], wo, w1, w2, wave, lane);
-    mlp_ff_pstage<F16, 1>(lds[0], b1s, xb, u + 1, hh, lane, h, acc);
-  }
-  stage_barrier();
-  mlp_issue(s0 + kFfStages, lds[0], wo, w1, w2, wave, lane);
-  mlp_ff_pstage<F16, 1>(lds[1], b1s, xb, kFfStages - 1, hh, lane, h, acc);
-  stage_barrier();
-  mlp_ff_pstage<F16, 2>(lds[0], b1s, xb, kFfStages, hh, lane, h, acc);
-}
-
-template <bool OUTPROJ, bool FF, bool F16>
-__global__ __launch_bounds__(512) void k_mlp(const uint16_t* __restrict__ O, const uint8_t* __restrict__ layer,
-                                             float* __restrict__ X, uint16_t* __restrict__ xn, int64_t n, float eps) {
-  // One LDS object: 2 stages x 32 operand blocks of 1 KB, then b1 (4 KB) and b2 (1 KB).  (With a second
-  // __shared__ object written by direct-to-LDS loads, the compiler waits for those loads before every
-  // operand read.)
-  __shared__ u32x4 smem[2 * 32 * 64 + (kHidden + kDim) / 4];
-  u32x4 (*lds)[32 * 64] = reinterpret_cast<u32x4 (*)[32 * 64]>(smem);
-  u32x4* bias = smem + 2 * 32 * 64;
-  const u32x4* wo = reinterpret_cast<const u32x4*>(layer + kOffOut);
-  const u32x4* w1 = reinterpret_cast<const u32x4*>(layer + (F16 ? kOffFf1F16 : kOffFf1));
-  const u32x4* w2 = reinterpret_cast<const u32x4*>(layer + (F16 ? kOffFf2F16 : kOffFf2));
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int j = lane & 31, hh = lane >> 5;
-  const int64_t tok = (int64_t(blockIdx.x) * kMlpWaves + wave) * 32 + j;
-  // Lanes past the last token work on a copy of the last token's row (every MFMA column and the
-  // half-wave norm swap stay within one token) and store nothing.
-  const bool valid = tok < n;
-  const int64_t trow = valid ? tok : n - 1;
-  float* xr = X + trow * kDim;
-  uint16_t* nr = xn + trow * kDim;
-
-  // With the out-projection, X joins the accumulators one 32-row tile per stage (its loads spread over
-  // the stages instead of all waves of the chip loading it at once); without it, they start at X.
-  f32x16 acc[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 x = OUTPROJ ? f32x4{0.f, 0.f, 0.f, 0.f}
-                              : *reinterpret_cast<const f32x4*>(xr + 32 * t + row_of_group(g, hh));
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[t][4 * g + r] = x[r];
-    }
-
-  constexpr int s_begin = OUTPROJ ? 0 : kOutStages;
-  constexpr int s_end = FF ? kOutStages + kFfStages + 1 : kOutStages;
-  if (FF && wave < 4)  // b1 (4 KB) and b2 (1 KB) into LDS; the first stage barrier waits for them
-    lds_load_block(reinterpret_cast<const u32x4*>(layer + kOffBff1) + wave * 64, &bias[wave * 64], lane);
-  if (FF && wave == 4) lds_load_block(reinterpret_cast<const u32x4*>(layer + kOffBff2), &bias[kHidden / 4], lane);
-  mlp_issue(s_begin, lds[0], wo, w1, w2, wave, lane);
-  if (OUTPROJ) {
-    const uint16_t* orow = O + trow * 512;
-    u32x4 ob[4];  // O operands of the next stage
-    auto load_o = [&](int s) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ob[i] = reinterpret_cast<const u32x4*>(orow)[2 * (4 * s + i) + hh];
-    };
-    f32x4 xt[4];  // X tile of the next stage
-    auto load_x = [&](int t) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) xt[g] = *reinterpret_cast<const f32x4*>(xr + 32 * t + row_of_group(g, hh));
-    };
-    load_o(0);
-    load_x(0);
-#pragma unroll
-    for (int s = 0; s < kOutStages; ++s) {
-      stage_barrier();
-      if (s + 1 < s_end) mlp_issue(s + 1, lds[(s + 1) & 1], wo, w1, w2, wave, lane);
-      const u32x4 cur[4] = {ob[0], ob[1], ob[2], ob[3]};
-      const f32x4 xs[4] = {xt[0], xt[1], xt[2], xt[3]};
-      if (s + 1 < kOutStages) {
-        load_o(s + 1);
-        load_x(s + 1);
-      }
-      mlp_out_block(lds[s & 1], cur, lane, acc);
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[s][4 * g + r] += xs[g][r];
-    }
-  }
-  const float inv = acc_inv_norm(acc, eps);
-  if (!FF) {
-    if (valid) store_row(acc, inv, xr, nr, hh);
-    return;
-  }
-  u32x4 xb[16];  // FF1 B operands: xn = X / |X| in register order, bf16 or fp16
-#pragma unroll
-  for (int ks = 0; ks < 16; ++ks) {
-    const int t = ks >> 1, g0 = 2 * (ks & 1);
-    xb[ks] = u32x4{pk_ff<F16>(acc[t][4 * g0] * inv, acc[t][4 * g0 + 1] * inv),
-                   pk_ff<F16>(acc[t][4 * g0 + 2] * inv, acc[t][4 * g0 + 3] * inv),
-                   pk_ff<F16>(acc[t][4 * g0 + 4] * inv, acc[t][4 * g0 + 5] * inv),
-                   pk_ff<F16>(acc[t][4 * g0 + 6] * inv, acc[t][4 * g0 + 7] * inv)};
-  }
-  const f32x4* bf = reinterpret_cast<const f32x4*>(bias);
-  mlp_ff_stages<F16>(acc, xb, lds, bf, wo, w1, w2, wave, lane, hh);
-#pragma unroll
-  for (int t = 0; t < 8; ++t)  // + b2
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 b = bf[kHidden / 4 + 8 * t + 2 * g + hh];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[t][4 * g + r] += b[r];
-    }
-  const float inv2 = acc_inv_norm(acc, eps);
-  if (valid) store_row(acc, inv2, xr, nr, hh);
-}
-
-// ============================================================ split-bf16 feed-forward
-// Both FF GEMMs take split-bf16 operands v = hi + lo (hi = bf16(v), lo = bf16(v - hi)) and form
-// hi.hi + hi.lo + lo.hi on the bf16 MFMA with fp32 accumulation; the dropped lo.lo term is ~2^-16
-// relative.  xn and the GELU output are split in registers, W1 and W2 carry packed lo parts, and the
-// out-projection stays bf16.  These four operands (W1, W2, xn into FF1, gelu(h)) are the rounding
-// points that dominate the error of the all-bf16 design.
+// The accumulator registers of a 32-row tile are the B operand of two k-steps as they stand (W1, W2 are
+// packed in register order), so xn1 and gelu(h) pass through LDS as whole operand blocks, and the
+// 1024-wide hidden activation never leaves the chip.  FF1 of block c + 1 comes before FF2 of block c, whose
+// MFMAs the GELU of block c + 1 is spread between.
+// The feed-forward runs in bf16, fp16 or split-bf16 operands (PREC, FfPrecision); the out-projection stays
+// bf16.  Split: both FF GEMMs take v = hi + lo (hi = bf16(v), lo = bf16(v - hi)) and form
+// hi.hi + hi.lo + lo.hi with fp32 accumulation; the dropped lo.lo term is ~2^-16 relative.
+// Without OUTPROJ the block starts at X (the feed-forward sub-layer alone); xn may be null (not written).
 //
-// Shape: v_mfma_f32_16x16x32_bf16 with 16 tokens per wave (output features on the 16 rows, tokens on
-// the 16 columns; lane l holds token l%16 and rows 4(l/16)..+3 of a tile).  The residual stream is 16
-// tiles x 4 registers and the hi and lo B operands of xn 2 x 32 registers, so a wave fits in 256
-// registers and two waves share each SIMD: one wave's GELU runs while the other's MFMAs do.  A
-// workgroup is 4 waves (64 tokens) with 2 x 32 KB of LDS stages, two workgroups per CU.
-// Stages: 0..7 out-projection (W_out k-steps 2s, 2s+1 of all 16 tiles); then for each block j of 32
-// hidden units, stage A_j = W1 hi and lo of tiles 2j, 2j+1 (FF1), and stage B_j = W2 hi and lo of
-// k-step j of all 16 output tiles (GELU of block j, FF2).
-constexpr int kX3Waves = 4;
-constexpr int kX3OutStages = 8;
-constexpr int kX3Blocks = kHidden / 32;
-constexpr int kX3Stages = kX3OutStages + 2 * kX3Blocks;
+// What it replaced: 256-token workgroups whose waves each held all 256 features of 32 tokens and took the
+// weights from LDS in 41 barrier-separated stages (fp16, bf16), and the same with 16 tokens a wave on
+// 16x16x32 MFMAs (split).  us per launch, then and now: 212 and 180 at 105,462 tokens in the stack (fp16),
+// 80 and 21.5 at 6,262; the feed-forward alone 74 and 38 at 18,786 (fp16), 365 and 319 at 105,462 (split).
+// At 105,462 tokens the parts are 74 us of HBM traffic (378 MB at the rate of a copy), 56 us of MFMA work
+// and, without either, ~30 us for the weights' way from L2; the tiles of a round start together, so they
+// overlap only in part (priorities for one of a CU's two workgroups change nothing).
+// (fast.py:311-331, kernels.cpp:542-642)
 
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                 0, 0, 0);
+// FF operand packing and products of the one-part arithmetics.
+template <int PREC>
+__device__ __forceinline__ uint32_t pk_ff(float lo, float hi) {
+  return PREC == kFfFp16 ? pk_f16(lo, hi) : pk_bf16(lo, hi);
 }
-
-__device__ __forceinline__ f32x4 zero4f() {
-  f32x4 z = {};
-  return z;
+template <int PREC>
+__device__ __forceinline__ f32x16 mfma_ff(u32x4 a, u32x4 b, f32x16 c) {
+  return PREC == kFfFp16 ? mfma32h(a, b, c) : mfma32(a, b, c);
 }
+__host__ __device__ constexpr int ff_parts(int prec) { return prec == kFfSplit ? 2 : 1; }
 
+// The bf16 hi and lo parts of a pair.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
   hi = pk_bf16(a, b);
   lo = pk_bf16(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u));
 }
 
-// Register-order B operand from two 16x16 accumulator tiles (values scaled by s): element pairs
-// (tile u, rows 2q', 2q'+1) in the order of kperm16 = 16(e/4) + 4g + e%4.
-__device__ __forceinline__ void split_operand(const f32x4& t0, const f32x4& t1, float s, u32x4& hi, u32x4& lo) {
-  uint32_t h, l;
-  split_pair(t0[0] * s, t0[1] * s, h, l);
-  hi[0] = h;
-  lo[0] = l;
-  split_pair(t0[2] * s, t0[3] * s, h, l);
-  hi[1] = h;
-  lo[1] = l;
-  split_pair(t1[0] * s, t1[1] * s, h, l);
-  hi[2] = h;
-  lo[2] = l;
-  split_pair(t1[2] * s, t1[3] * s, h, l);
-  hi[3] = h;
-  lo[3] = l;
+// Operand pair (a, b) of an FF GEMM into word q of the part's operand registers.
+template <int PREC>
+__device__ __forceinline__ void pack_ff(float a, float b, u32x4 (&v)[ff_parts(PREC)], int q) {
+  if constexpr (PREC == kFfSplit) {
+    uint32_t h, l;
+    split_pair(a, b, h, l);
+    v[0][q] = h;
+    v[1][q] = l;
+  } else {
+    v[0][q] = pk_ff<PREC>(a, b);
+  }
 }
 
-struct X3Weights {
-  const u32x4* wo;   // W_out, 16x16 natural: [16 tiles][16 k-steps]
-  const u32x4* w1h;  // W1 hi / lo, 16x16 register order: [64 tiles][8 k-steps]
-  const u32x4* w1l;
-  const u32x4* w2h;  // W2 hi / lo, 16x16 register order: [16 tiles][32 k-steps]
-  const u32x4* w2l;
+// A wave's stream of weight blocks: k-step k of the current GEMM is at off[part] + k KB of the layer.
+struct PaWeights {
+  __amdgpu_buffer_rsrc_t res;
+  int lane16;
+  __device__ __forceinline__ u32x4 load(int off) const { return buffer_load16(res, lane16, off); }
 };
 
-// This wave's 8 of the stage's 32 blocks into LDS buffer dst.
-__device__ __forceinline__ void x3_issue(const X3Weights& w, int s, u32x4* dst, int wave, int lane) {
+// acc += W . B over KS k-steps.  a holds the first kWeightAhead k-steps' blocks and is left with those of
+// the next GEMM (at next[], NEXT parts; 0: there is none).  b(k, part, ct) is the LDS operand.  side(k) is
+// VALU work placed beside k-step k's MFMAs.
+template <int KS, int C, int PREC, int NEXT, typename Operand, typename Side>
+__device__ __forceinline__ void pa_gemm(const PaWeights& w, const int (&off)[2], const int (&next)[2],
+                                        u32x4 (&a)[kWeightAhead][2], f32x16 (&acc)[C], Operand&& operand,
+                                        Side&& side) {
+  constexpr int NP = ff_parts(PREC);
+  constexpr int AHEAD = C == 1 ? (NP == 1 ? 4 : 2) : 1;  // k-steps the activation operands are read ahead
+  u32x4 b[AHEAD + 1][NP][C];
+  auto read = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int b = wave * 8 + i;
-    const u32x4* src;
-    if (s < kX3OutStages) {
-      src = w.wo + (int64_t(b >> 1) * 16 + 2 * s + (b & 1)) * 64;  // tile b/2, k-step 2s + b%2
-    } else {
-      const int u = s - kX3OutStages, j = u >> 1;
-      if ((u & 1) == 0)  // A_j: part b/16 (hi, lo), tile 2j + (b/8)%2, k-step b%8
-        src = ((b < 16) ? w.w1h : w.w1l) + (int64_t(2 * j + ((b >> 3) & 1)) * 8 + (b & 7)) * 64;
-      else  // B_j: part b/16, output tile b%16, k-step j
-        src = ((b < 16) ? w.w2h : w.w2l) + (int64_t(b & 15) * 32 + j) * 64;
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) b[k % (AHEAD + 1)][p][ct] = operand(k, p, ct);
+  };
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) read(k);
+#pragma unroll
+  for (int k = 0; k < KS; ++k) {
+    if (k + AHEAD < KS) read(k + AHEAD);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 (&ak)[2] = a[k % kWeightAhead];
+    u32x4 (&bk)[NP][C] = b[k % (AHEAD + 1)];
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[0], bk[0][ct], acc[ct]);
+    if constexpr (NP == 2) {
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[0], bk[1][ct], acc[ct]);
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[1], bk[0][ct], acc[ct]);
     }
-    lds_load_block(src, dst + b * 64, lane);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      if (k + kWeightAhead < KS) {
+        if (p < NP) ak[p] = w.load(off[p] + (k + kWeightAhead) * kTileBytes);
+      } else if (p < NEXT) {
+        ak[p] = w.load(next[p] + (k + kWeightAhead - KS) * kTileBytes);
+      }
+    }
+    side(k);
+    __builtin_amdgcn_sched_barrier(0);
   }
+  // The products end here: without this the compiler may sink the whole MFMA chain, whose only readers come
+  // later, past the next barrier, and keep every operand in scratch until then.
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct) asm volatile("" : "+v"(acc[ct]));
 }
 
-template <bool OUTPROJ>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mlp_x3(
+// The split arithmetic at C = 2 holds 128 KB of operands: one workgroup per CU, 256 registers a wave.
+constexpr int pa_waves_per_simd(int C, int prec) { return C == 2 && prec == kFfSplit ? 2 : 4; }
+
+template <int C, bool OUTPROJ, int PREC>
+__global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k_post_attn(
     const uint16_t* __restrict__ O, const uint8_t* __restrict__ layer, float* __restrict__ X,
     uint16_t* __restrict__ xn, int64_t n, float eps) {
-  __shared__ u32x4 lds[2][32 * 64];  // 2 stages x 32 operand blocks of 1 KB
-  X3Weights w;
-  w.wo = reinterpret_cast<const u32x4*>(layer + kOffOut16);
-  w.w1h = reinterpret_cast<const u32x4*>(layer + kOffFf1Hi16);
-  w.w1l = reinterpret_cast<const u32x4*>(layer + kOffFf1Lo16);
-  w.w2h = reinterpret_cast<const u32x4*>(layer + kOffFf2Hi16);
-  w.w2l = reinterpret_cast<const u32x4*>(layer + kOffFf2Lo16);
-  const float* b1 = reinterpret_cast<const float*>(layer + kOffBff1);
-  const float* b2 = reinterpret_cast<const float*>(layer + kOffBff2);
+  constexpr int R = 32 * C, RW = R / kTileWaves;  // tokens of the tile, rows a wave moves
+  constexpr int NP = ff_parts(PREC);
+  constexpr int kPart = C * 16 * 64;  // one part of xn1 or of a hidden block as operand blocks [ct][k-step][lane]
+  constexpr int kBias = 2 * NP * kPart, kSsq = kBias + (kHidden + kDim) / 4;
+  __shared__ u32x4 smem[kSsq + R * kTileWaves / 4];
+  u32x4* const xb = smem;               // xn1; with hb also the tile's O rows, X rows and output rows
+  u32x4* const hb = smem + NP * kPart;  // gelu(h) of one block
+  const u32x4* const bias = smem + kBias;  // b1, b2
+  float* const ssq = reinterpret_cast<float*>(smem + kSsq);
   const int lane = threadIdx.x & 63, wave = wave_id();
-  const int col = lane & 15, g = lane >> 4;
-  const int64_t tok = (int64_t(blockIdx.x) * kX3Waves + wave) * 16 + col;
-  const bool valid = tok < n;  // lanes past the end work on the last token's row and store nothing
-  const int64_t trow = valid ? tok : n - 1;
-  float* xr = X + trow * kDim;
-  uint16_t* nr = xn + trow * kDim;
-
-  f32x4 acc[16];  // residual stream: tile t holds features 16t + 4g + r of this lane's token
-#pragma unroll
-  for (int t = 0; t < 16; ++t) acc[t] = *reinterpret_cast<const f32x4*>(xr + 16 * t + 4 * g);
-
-  auto inv_norm = [&]() __attribute__((always_inline)) {
-    float ss = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ss = fmaf(acc[t][r], acc[t][r], ss);
-    ss += __shfl_xor(ss, 16);
-    ss += __shfl_xor(ss, 32);
-    return 1.0f / fmaxf(sqrtf(ss), eps);
-  };
-
-  int s0 = OUTPROJ ? 0 : kX3OutStages;
-  x3_issue(w, s0, lds[0], wave, lane);
-  if (OUTPROJ) {
-    const u32x4* orow = reinterpret_cast<const u32x4*>(O + trow * 512);
-    u32x4 ob[2] = {orow[g], orow[4 + g]};  // k-steps 0, 1: O features 32ks + 8g..+7
-    for (int s = 0; s < kX3OutStages; ++s) {
-      stage_barrier();
-      x3_issue(w, s + 1, lds[(s + 1) & 1], wave, lane);
-      const u32x4* Ls = lds[s & 1];
-      const u32x4 cur[2] = {ob[0], ob[1]};
-      if (s + 1 < kX3OutStages) {
-        ob[0] = orow[4 * (2 * s + 2) + g];
-        ob[1] = orow[4 * (2 * s + 3) + g];
-      }
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-        for (int t = 0; t < 16; ++t) acc[t] = mfma16(Ls[(2 * t + kk) * 64 + lane], cur[kk], acc[t]);
-    }
-  }
-  u32x4 xb[8], xl[8];  // FF1 B operands: xn hi and lo, k-step ks = tiles 2ks, 2ks+1 in register order
+  const int j = lane & 31, hh = lane >> 5, t0 = wave * RW;
+  const int64_t tok0 = int64_t(blockIdx.x) * R;
+  const int rows = int(n - tok0 < R ? n - tok0 : R);  // rows past the last token read as zeros, stores drop
+  const auto xres = buffer_rsrc(X + tok0 * kDim, rows * kDim * 4);
+  const auto nres = buffer_rsrc(xn + tok0 * kDim, xn ? rows * kDim * 2 : 0);
+  const PaWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
   {
-    const float inv = inv_norm();
+    static_assert(kDim * 4 == 512 * 2, "rows of O and X are 1 KB");
+    const auto rres = OUTPROJ ? buffer_rsrc(O + tok0 * 512, rows * 1024) : xres;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) split_operand(acc[2 * ks], acc[2 * ks + 1], inv, xb[ks], xl[ks]);
+    for (int i = 0; i < RW; ++i)
+      buffer_load_lds16(rres, (t0 + i) * 1024 + 16 * (lane ^ ((t0 + i) & 15)), smem + (t0 + i) * 64);
+    if (wave < 4) buffer_load_lds16(w.res, int(kOffBff1) + wave * 1024 + lane * 16, smem + kBias + wave * 64);
+    if (wave == 4) buffer_load_lds16(w.res, int(kOffBff2) + lane * 16, smem + kBias + kHidden / 4);
+  }
+  u32x4 xr[RW];  // X rows, added after the out-projection
+  if (OUTPROJ) {
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(b2 + 16 * t + 4 * g);
-      acc[t] += b;
+    for (int i = 0; i < RW; ++i) xr[i] = buffer_load16(xres, lane * 16 + (t0 + i) * 1024, 0);
+  }
+  constexpr int w1[2] = {int(PREC == kFfFp16 ? kOffFf1F16 : kOffFf1), int(kOffFf1Lo)};
+  constexpr int w2[2] = {int(PREC == kFfFp16 ? kOffFf2F16 : kOffFf2), int(kOffFf2Lo)};
+  struct Off {
+    int v[2];
+  };
+  const Off out{{int(kOffOut) + wave * 32 * kTileBytes, 0}};
+  auto ff1 = [&](int c) __attribute__((always_inline)) { return Off{{w1[0] + (8 * c + wave) * 16 * kTileBytes, w1[1] + (8 * c + wave) * 16 * kTileBytes}}; };
+  auto ff2 = [&](int c) __attribute__((always_inline)) { return Off{{w2[0] + (64 * wave + 16 * c) * kTileBytes, w2[1] + (64 * wave + 16 * c) * kTileBytes}}; };
+  u32x4 a[kWeightAhead][2];
+  {
+    const Off first = OUTPROJ ? out : ff1(0);
+#pragma unroll
+    for (int i = 0; i < kWeightAhead; ++i)
+#pragma unroll
+      for (int p = 0; p < (OUTPROJ ? 1 : NP); ++p) a[i][p] = w.load(first.v[p] + i * kTileBytes);
+  }
+  auto none = [](int) __attribute__((always_inline)) {};
+  f32x16 acc[C];
+  loads_barrier();
+  if (OUTPROJ) {
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
+    const int m = j & 15, base = j * 64 + (hh ^ (m & 1)), me = m & 14;  // chunk 2k + hh of token j
+    pa_gemm<32, C, kFfBf16, NP>(w, out.v, ff1(0).v, a, acc,
+                                [&](int k, int, int ct) __attribute__((always_inline)) {
+                                  return smem[base + ((2 * k) ^ me) + ct * 32 * 64];
+                                },
+                                none);
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < RW; ++i) smem[row_chunk(t0 + i, lane)] = xr[i];
+    lds_barrier();
+  }
+  add_rows<C, !OUTPROJ>(smem, acc, wave, j, hh);
+  put_ssq(acc, ssq, wave, j, hh);
+  lds_barrier();
+#pragma unroll
+  for (int ct = 0; ct < C; ++ct) {
+    const float inv = inv_norm(ssq, 32 * ct + j, eps);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      u32x4 v[NP];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pack_ff<PREC>(acc[ct][8 * q + 2 * e] * inv, acc[ct][8 * q + 2 * e + 1] * inv, v, e);
+#pragma unroll
+      for (int p = 0; p < NP; ++p) xb[p * kPart + (ct * 16 + 2 * wave + q) * 64 + lane] = v[p];
     }
   }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const f32x4 b = __builtin_bit_cast(f32x4, bias[kHidden / 4 + 8 * wave + 2 * g + hh]);
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[ct][4 * g + r] += b[r];
+  }
+  lds_barrier();
 
-  f32x4 hs[2];  // FF1 of the current hidden block (tiles 2j, 2j+1), before bias and GELU
-  for (int j = 0; j < kX3Blocks; ++j) {
-    const int s = kX3OutStages + 2 * j;
-    // stage A_j: FF1 of hidden tiles 2j, 2j+1
-    stage_barrier();
-    x3_issue(w, s + 1, lds[(s + 1) & 1], wave, lane);
-    {
-      const u32x4* Ls = lds[s & 1];
-      f32x4 h0[2] = {zero4f(), zero4f()}, h1[2] = {zero4f(), zero4f()};
+  f32x16 h[C];
+  u32x4 hp[C][2][NP];  // gelu(h) as operands
+  auto start_h = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks)
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = __builtin_bit_cast(f32x4, bias[8 * (8 * c + wave) + 2 * g + hh]);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const u32x4 a = Ls[(8 * u + ks) * 64 + lane], al = Ls[(16 + 8 * u + ks) * 64 + lane];
-          h0[u] = mfma16(a, xb[ks], h0[u]);
-          h1[u] = mfma16(a, xl[ks], h1[u]);
-          h0[u] = mfma16(al, xb[ks], h0[u]);
-        }
-      hs[0] = h0[0] + h1[0];
-      hs[1] = h0[1] + h1[1];
+      for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) h[ct][4 * g + r] = b[r];
     }
-    // stage B_j: GELU of block j, then FF2 k-step j into every output tile
-    const f32x4 bb0 = *reinterpret_cast<const f32x4*>(b1 + 32 * j + 4 * g);
-    const f32x4 bb1 = *reinterpret_cast<const f32x4*>(b1 + 32 * j + 16 + 4 * g);
-    stage_barrier();
-    if (s + 2 < kX3Stages) x3_issue(w, s + 2, lds[s & 1], wave, lane);
-    {
-      const u32x4* Ls = lds[(s + 1) & 1];
-      f32x4 v0, v1;
+  };
+  auto gelu_pair = [&](int v) __attribute__((always_inline)) {  // values 2v, 2v + 1 of the wave's 16 C per lane
+    const int ct = v >> 3, p = v & 7;
+    const float x = h[ct][2 * p], y = h[ct][2 * p + 1];
+    if constexpr (PREC == kFfSplit)
+      pack_ff<PREC>(gelu_erf(x), gelu_erf(y), hp[ct][p >> 2], p & 3);
+    else
+      pack_ff<PREC>(gelu_logistic(x), gelu_logistic(y), hp[ct][p >> 2], p & 3);
+  };
+  auto put_h = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v0[r] = gelu_erf(hs[0][r] + bb0[r]);
-        v1[r] = gelu_erf(hs[1][r] + bb1[r]);
-      }
-      u32x4 hb, hl;
-      split_operand(v0, v1, 1.0f, hb, hl);
+    for (int ct = 0; ct < C; ++ct)
 #pragma unroll
-      for (int t = 0; t < 16; ++t) {
-        const u32x4 a = Ls[t * 64 + lane], al = Ls[(16 + t) * 64 + lane];
-        acc[t] = mfma16(a, hb, acc[t]);
-        acc[t] = mfma16(a, hl, acc[t]);
-        acc[t] = mfma16(al, hb, acc[t]);
-      }
-    }
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int p = 0; p < NP; ++p) hb[p * kPart + (ct * 16 + 2 * wave + q) * 64 + lane] = hp[ct][q][p];
+    lds_barrier();
+  };
+  auto xop = [&](int k, int p, int ct) __attribute__((always_inline)) { return xb[p * kPart + (ct * 16 + k) * 64 + lane]; };
+  auto hop = [&](int k, int p, int ct) __attribute__((always_inline)) { return hb[p * kPart + (ct * 16 + k) * 64 + lane]; };
+  constexpr int kBlocks = kHidden / 256;
+  start_h(0);
+  pa_gemm<16, C, PREC, NP>(w, ff1(0).v, ff1(1).v, a, h, xop, none);
+#pragma unroll
+  for (int v = 0; v < 8 * C; ++v) gelu_pair(v);
+  put_h();
+#pragma unroll
+  for (int c = 1; c < kBlocks; ++c) {
+    start_h(c);
+    pa_gemm<16, C, PREC, NP>(w, ff1(c).v, ff2(c - 1).v, a, h, xop, none);
+    pa_gemm<16, C, PREC, NP>(w, ff2(c - 1).v, (c + 1 < kBlocks ? ff1(c + 1) : ff2(c)).v, a, acc, hop,
+                             [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+                               for (int v = k * C / 2; v < (k + 1) * C / 2; ++v) gelu_pair(v);
+                             });
+    lds_barrier();  // every wave has read block c - 1
+    put_h();
   }
-  const float inv = inv_norm();
-  if (valid) {
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      *reinterpret_cast<f32x4*>(xr + 16 * t + 4 * g) = acc[t];
-      const u32x2 v = {pk_bf16(acc[t][0] * inv, acc[t][1] * inv), pk_bf16(acc[t][2] * inv, acc[t][3] * inv)};
-      *reinterpret_cast<u32x2*>(nr + 16 * t + 4 * g) = v;
-    }
-  }
+  pa_gemm<16, C, PREC, 0>(w, ff2(kBlocks - 1).v, out.v, a, acc, hop, none);
+  put_ssq(acc, ssq, wave, j, hh);
+  lds_barrier();
+  store_tile(acc, smem, ssq, eps, xres, nres, wave, lane);
 }
 
-void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, bool with_ff,
-                      int ff_precision, float eps, hipStream_t st, const LaunchEvents& ev) {
-  if (with_ff && ff_precision == kFfSplit) {
-    const unsigned blocks = unsigned((n + 16 * kX3Waves - 1) / (16 * kX3Waves));
-    hipExtLaunchKernelGGL(k_mlp_x3<true>, dim3(blocks), dim3(64 * kX3Waves), 0, st, ev.start, ev.stop, 0, O, layer, X,
-                          xn, n, eps);
-    return;
-  }
-  const unsigned blocks = unsigned((n + 32 * kMlpWaves - 1) / (32 * kMlpWaves));
-  if (!with_ff)
-    hipExtLaunchKernelGGL((k_mlp<true, false, false>), dim3(blocks), dim3(64 * kMlpWaves), 0, st, ev.start, ev.stop, 0, O, layer,
-                          X, xn, n, eps);
-  else if (ff_precision == kFfFp16)
-    hipExtLaunchKernelGGL((k_mlp<true, true, true>), dim3(blocks), dim3(64 * kMlpWaves), 0, st, ev.start, ev.stop, 0, O, layer,
-                          X, xn, n, eps);
-  else
-    hipExtLaunchKernelGGL((k_mlp<true, true, false>), dim3(blocks), dim3(64 * kMlpWaves), 0, st, ev.start, ev.stop, 0, O, layer,
-                          X, xn, n, eps);
+namespace {
+template <bool OUTPROJ>
+void launch_block(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int prec, float eps,
+                  hipStream_t st, const LaunchEvents& ev) {
+  const int C = token_tiles(n);
+  const auto kernel =
+      prec == kFfSplit  ? (C == 1 ? k_post_attn<1, OUTPROJ, kFfSplit> : k_post_attn<2, OUTPROJ, kFfSplit>)
+      : prec == kFfFp16 ? (C == 1 ? k_post_attn<1, OUTPROJ, kFfFp16> : k_post_attn<2, OUTPROJ, kFfFp16>)
+                        : (C == 1 ? k_post_attn<1, OUTPROJ, kFfBf16> : k_post_attn<2, OUTPROJ, kFfBf16>);
+  hipExtLaunchKernelGGL(kernel, dim3(unsigned((n + 32 * C - 1) / (32 * C))), dim3(64 * kTileWaves), 0, st, ev.start,
+                        ev.stop, 0, O, layer, X, xn, n, eps);
+}
+}  // namespace
+
+void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision,
+                      float eps, hipStream_t st, const LaunchEvents& ev) {
+  launch_block<true>(O, layer, X, xn, n, ff_precision, eps, st, ev);
 }
 
 void launch_ff(const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision, float eps, hipStream_t st) {
-  const uint16_t* none = nullptr;
-  if (ff_precision == kFfSplit) {
-    const unsigned blocks = unsigned((n + 16 * kX3Waves - 1) / (16 * kX3Waves));
-    hipLaunchKernelGGL(k_mlp_x3<false>, dim3(blocks), dim3(64 * kX3Waves), 0, st, none, layer, X, xn, n, eps);
-    return;
-  }
-  const unsigned blocks = unsigned((n + 32 * kMlpWaves - 1) / (32 * kMlpWaves));
-  if (ff_precision == kFfFp16)
-    hipLaunchKernelGGL((k_mlp<false, true, true>), dim3(blocks), dim3(64 * kMlpWaves), 0, st, none, layer, X, xn, n, eps);
-  else
-    hipLaunchKernelGGL((k_mlp<false, true, false>), dim3(blocks), dim3(64 * kMlpWaves), 0, st, none, layer, X, xn, n, eps);
+  launch_block<false>(nullptr, layer, X, xn, n, ff_precision, eps, st, LaunchEvents{});
 }
 
 }  // namespace trf
