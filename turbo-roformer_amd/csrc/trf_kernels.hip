@@ -11,7 +11,7 @@
 // Numerics follow the reference kernels (src/turbo_roformer/csrc/kernels.cpp): fp32
 // accumulators, fp32 residual stream, fp32 rotary/softmax/gate math, bf16 round-to-nearest-even
 // for every GEMM/attention operand (kernels.cpp:30-33).
-#include "trf_device.h"
+#include "trf_tiles.h"
 
 #include <atomic>
 
@@ -135,212 +135,119 @@ void launch_add_rmsnorm(float* X, const void* Y, int y_bf16, void* out, int out_
 }
 
 // ============================================================ fused QKV + gate GEMM, rotary epilogue
-// One wave owns 32 consecutive padded positions of one sequence; its 32 tokens' xn rows stay in
-// registers as B operands.  The workgroup (8 waves, 2 per SIMD) streams the 49 weight tiles through
-// LDS four per stage (13 stages: q heads, k heads, v heads, then the gate tile), so every stage is of
-// one kind.  The rotary cos/sin of the wave's position is loaded into registers with its xn rows.
+// A workgroup is 32 C consecutive padded positions of one sequence; wave h computes head h: its q, k and v
+// weight tiles (two 32-row tiles each) one after the other, from L2 into registers, against the xn rows in
+// LDS (see trf_tiles.h).  The accumulators of a tile leave at once:
+//   q, k: rotated in fp32 (cos / sin rows of the tile's positions in LDS), packed; the half-waves trade
+//     register groups so that a lane stores a whole 16-byte chunk (8 features) of its position and an
+//     instruction writes two runs of 512 bytes (chunk-major rows, see token-order contract in trf_hip.h);
+//   v: the operands of the product are swapped, so a lane holds one feature of 4 consecutive positions per
+//     register group; V^T rows go through the wave's own 8 KB of LDS and leave as whole lines.
+// The gate tile's 16 k-steps are split over the waves (two each) and summed through LDS.
+// Bounded by the writes: 324 MB of Q, K, V^T at 105,462 tokens (68 us at the rate of 8-byte store streams).
+// Workgroups of 256 rows that streamed the weights through LDS in 13 barrier-separated stages and stored
+// 8 bytes a lane took 22.6 us at 101 frames x 62 bands (31 workgroups' rows on 256 CUs), 49 at 487 frames and
+// 134 at 1701; these take 15, 34 and 129.  What is left at 1701 is the L2's: a tile's weights pass once per 64
+// positions (the CUs' address units are 70% busy, waiting on it half of that time).
 // (kernels.cpp:439-540)
-//
-// A stage runs as two groups of two tiles (two interleaved MFMA chains each).  A group's outputs
-// leave as 8 packed 8-byte stores per lane, issued during the NEXT group's MFMA loop, one every other
-// k-step, so the write stream runs under the matrix work instead of in a burst between stages.  Stage
-// barriers wait with an exact vmcnt for the weight loads issued before those stores.
-//
-// Work is dealt in units of (block of 256 rows, stage): workgroup b of G runs units [bU/G, (b+1)U/G) of
-// the U = 13 x blocks in order, so one workgroup per CU gets an even share of stages (21 or 22 for the
-// 419 blocks of a 17 s chunk's time sub-layer) instead of two rounds of whole blocks (1.64 per CU).  A
-// block entered mid-way loads its xn rows and rotary table again; one left early stores its last group
-// at once.
-constexpr int kQkvWaves = 8;
-constexpr int kQkvTps = 4;
-constexpr int kQkvStages = (kQkvgTiles + kQkvTps - 1) / kQkvTps;
-constexpr int kQkvGroupStores = 8;  // 2 tiles x 4 register groups
-
-__global__ __launch_bounds__(512) void k_qkv_rope(const uint16_t* __restrict__ xn, const u32x4* __restrict__ wq,
-                                                  const float* __restrict__ bgate, const float* __restrict__ rope,
-                                                  int mode, int nseq, int L, int Lpad, int T, int F, int nblocks,
-                                                  uint16_t* __restrict__ Q, uint16_t* __restrict__ K,
-                                                  uint16_t* __restrict__ Vt, float* __restrict__ G) {
-  __shared__ u32x4 lds[2][kQkvTps * 16 * 64];  // 2 stages x 4 tiles x 16 k-steps x 1 KB
+template <int C>
+__global__ __launch_bounds__(64 * kTileWaves, 4) void k_qkv_rope(
+    const uint16_t* __restrict__ xn, const uint8_t* __restrict__ layer, const float* __restrict__ rope, int mode,
+    int L, int Lpad, int T, int F, uint16_t* __restrict__ Q, uint16_t* __restrict__ K, uint16_t* __restrict__ Vt,
+    float* __restrict__ G) {
+  constexpr int R = 32 * C;
+  constexpr int kRope = R * 32, kGate = kRope + R * kRopeChunks;
+  __shared__ u32x4 smem[kGate + kTileWaves * R * kHeads / 4];  // xn blocks, cos | sin rows, partial gates; then V^T
+  static_assert(kGate + kTileWaves * R * kHeads / 4 >= kTileWaves * kHeadDim * R / 8, "V^T of the tile fits");
   const int lane = threadIdx.x & 63, wave = wave_id();
-  const int j = lane & 31, hh = lane >> 5;
-  const int units = nblocks * kQkvStages;
-  const int u_begin = int(int64_t(blockIdx.x) * units / gridDim.x);
-  const int u_end = int(int64_t(blockIdx.x + 1) * units / gridDim.x);
-  const int qd = lane & 3;
-
-  auto issue = [&](int stage, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int b = wave * 8 + i;  // 64 blocks per stage: tile 4*stage + b/16, k-step b%16
-      const int t = kQkvTps * stage + (b >> 4);
-      if (t < kQkvgTiles) lds_load_block(wq + (int64_t(t) * 16 + (b & 15)) * 64, &lds[buf][b * 64], lane);
-    }
+  const int j = lane & 31, hh = lane >> 5, h = wave;
+  const int nblk = Lpad / R, s = blockIdx.x / nblk, p0 = (blockIdx.x - s * nblk) * R;
+  const TileWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
+  auto tile = [&](int kind, int half) __attribute__((always_inline)) {  // kind 0 q, 1 k, 2 v
+    return TileOff{{int(kOffQkvg) + (16 * kind + 2 * h + half) * 16 * kTileBytes, 0}};
   };
-  issue(u_begin % kQkvStages, u_begin & 1);
-
-#pragma unroll 1
-  for (int u = u_begin; u < u_end;) {
-    const int blk = u / kQkvStages, st0 = u - blk * kQkvStages;
-    const int st1 = min(kQkvStages, st0 + (u_end - u));  // this block's stages st0 .. st1 - 1
-    const int64_t row0 = (int64_t(blk) * kQkvWaves + wave) * 32;
-    const bool active = row0 < int64_t(nseq) * Lpad;  // inactive waves still stage weights and meet barriers
-    const int s = active ? int(row0 / Lpad) : 0;
-    const int p = active ? int(row0 % Lpad) + j : 0;
-    const bool valid = active && p < L;
-    const int64_t tok = valid ? token_of(mode, s, p, T, F) : 0;
-
-    u32x4 bx[16];
-    {
-      const u32x4* xr = reinterpret_cast<const u32x4*>(xn + tok * kDim);
+  u32x4 a[kWeightAhead][2], ag[2];
 #pragma unroll
-      for (int ks = 0; ks < 16; ++ks) bx[ks] = valid ? xr[2 * ks + hh] : zero4();
-    }
-    // Rotary of this position: features d0 = 32 half + 8g + 4hh (+0..3) form the pairs
-    // i = 16 half + 4g + 2hh + c, c = 0, 1.  rope = [cos | sin] rows of 32.
-    float2 rc[2][4], rsn[2][4];
-    {
-      const float* cr = rope + int64_t(valid ? p : 0) * 32;
-      const float* sr = cr + int64_t(L) * 32;
+  for (int i = 0; i < kWeightAhead; ++i) a[i][0] = w.load(tile(0, 0).v[0] + i * kTileBytes);
 #pragma unroll
-      for (int half = 0; half < 2; ++half)
+  for (int i = 0; i < 2; ++i) ag[i] = w.load(int(kOffQkvg) + ((kQkvgTiles - 1) * 16 + 2 * wave + i) * kTileBytes);
+  TilePositions<C> x;
+  x.load(xn, mode, s, p0, L, T, F);
+  stage_rope<C>(rope, p0, L, smem + kRope);
+  x.put(smem);
+  lds_barrier();
+  gate_partials<C>(ag, smem, reinterpret_cast<float*>(smem + kGate), wave, lane);
+  lds_barrier();
+  {  // thread -> (position, head): 8 lanes write a token's 8 gates
+    const int p = threadIdx.x >> 3, head = threadIdx.x & 7;
+    if (p < R && p0 + p < L)
+      G[token_of(mode, s, p0 + p, T, F) * kHeads + head] = gate_of<C>(
+          reinterpret_cast<const float*>(smem + kGate), p, head,
+          reinterpret_cast<const float*>(layer + kOffBgate));
+  }
+  auto xop = [&](int k, int, int ct) __attribute__((always_inline)) { return smem[(ct * 16 + k) * 64 + lane]; };
+  auto none = [](int) __attribute__((always_inline)) {};
+  const int64_t head0 = (int64_t(s) * kHeads + h) * kHeadDim * Lpad;  // first element of this (sequence, head)
+#pragma unroll
+  for (int kind = 0; kind < 2; ++kind) {
+    const auto res = buffer_rsrc((kind ? K : Q) + head0, kHeadDim * Lpad * 2);
+    const float sc = kind ? 1.0f : kLog2e;  // q leaves in units of log2(e): scores are base-2 exponents
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      f32x16 acc[C];
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
+      tile_gemm<16, C, kFfBf16, 1>(w, tile(kind, half).v, (half ? tile(kind + 1, 0) : tile(kind, 1)).v, a, acc, xop, none);
+#pragma unroll
+      for (int ct = 0; ct < C; ++ct) {
+        const bool valid = p0 + 32 * ct + j < L;
+        u32x2 o[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          rc[half][g] = *reinterpret_cast<const float2*>(cr + 16 * half + 4 * g + 2 * hh);
-          rsn[half][g] = *reinterpret_cast<const float2*>(sr + 16 * half + 4 * g + 2 * hh);
+          o[g] = rotate_group(acc[ct], g, smem + kRope, 32 * ct + j, half, hh, sc);
+          if (!valid) o[g] = u32x2{0u, 0u};
         }
-    }
-
-    // q/k rows are chunk-major: features 8c..8c+7 of position p at ((s*8 + h)*8 + c)*Lpad + p, so the 32
-    // lanes of a half-wave store 32 consecutive 16-byte chunks (hh fills bytes 8hh..8hh+7).
-    const int64_t qk_off = (int64_t(s) * kHeads * 8 * Lpad + p) * 8 + 4 * hh;
-    // V^T rows: lane 4q + r of a half-wave stores row r of its register group at positions 4q..4q+3
-    const int64_t v_off = (int64_t(s) * kHeads * kHeadDim + 4 * hh + qd) * Lpad + (p & ~3);
-    u32x2 pend[kQkvGroupStores];  // the previous group's packed outputs
-
-    // Store i of the outputs of group grp of stage ps: tile 4ps + 2grp + i/4, register group i%4.  Every
-    // offset beyond the lane's own is wave-uniform.
-    auto store_pending = [&](int ps, int grp, int i) __attribute__((always_inline)) {
-      const int tt = 2 * grp + (i >> 2), g = i & 3, t = kQkvTps * ps + tt, half = tt & 1;
-      if (ps < 8) {
-        const int h = (t & 15) >> 1;
-        uint16_t* base = (ps < 4 ? Q : K) + qk_off;
-        const int64_t off = int64_t(__builtin_amdgcn_readfirstlane((h * 8 + 4 * half + g) * Lpad)) * 8;
-        *reinterpret_cast<u32x2*>(base + off) = pend[i];
-      } else {
-        const int h = (t - 32) >> 1;
-        const int drow = h * kHeadDim + 32 * half + 8 * g;  // row of V^T, less 4hh + r
-        *reinterpret_cast<u32x2*>(Vt + v_off + int64_t(__builtin_amdgcn_readfirstlane(drow * Lpad))) = pend[i];
-      }
-    };
-    // Everything loaded so far has landed (the block's first stage barrier waits for it anyway): stated
-    // as the builtin so that the compiler's own waitcnt insertion, which cannot tell the barrier branches
-    // below apart, adds no waits for the xn and rotary registers inside the stage loop.
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-#pragma unroll 1
-    for (int stage = st0; stage < st1; ++stage, ++u) {
-      // This stage's weight loads were issued at the top of the previous unit, whose two loops then
-      // issued 8 stores each (only the second loop in a block's first stage); a block's first stage
-      // follows the xn and rotary loads and waits for everything.
-      if (active && stage >= st0 + 2)
-        vmcnt_barrier<2 * kQkvGroupStores>();
-      else if (active && stage == st0 + 1)
-        vmcnt_barrier<kQkvGroupStores>();
-      else
-        vmcnt_barrier<0>();
-      if (u + 1 < u_end) issue((u + 1) % kQkvStages, (u + 1) & 1);
-      if (!active) continue;
-      const u32x4* Ls = lds[u & 1];
-      if (stage == kQkvStages - 1) {  // the gate tile: rows 0..7 live in register group 0 of both half-waves
-        f32x16 acc = zero16();
-        const bool pending = stage > st0;
 #pragma unroll
-        for (int ks = 0; ks < 16; ++ks) {
-          acc = mfma32(Ls[ks * 64 + lane], bx[ks], acc);
-          if ((ks & 1) && pending) store_pending(stage - 1, 1, ks >> 1);
-        }
-        if (valid) {
-          const f32x4 bg = *reinterpret_cast<const f32x4*>(bgate + 4 * hh);
-          f32x4 gv;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) gv[r] = 1.0f / (1.0f + expf(-(acc[r] + bg[r])));
-          *reinterpret_cast<f32x4*>(G + tok * kHeads + 4 * hh) = gv;
-        }
-        continue;
-      }
-#pragma unroll
-      for (int grp = 0; grp < 2; ++grp) {
-        f32x16 acc[2];
-        u32x4 a[2];
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          acc[v] = zero16();
-          a[v] = Ls[(2 * grp + v) * 16 * 64 + lane];
-        }
-        const bool pending = grp == 1 || stage > st0;
-#pragma unroll
-        for (int ks = 0; ks < 16; ++ks) {  // operands of k-step ks+1 are read while ks multiplies
-          u32x4 an[2];
-#pragma unroll
-          for (int v = 0; v < 2; ++v)
-            if (ks + 1 < 16) an[v] = Ls[((2 * grp + v) * 16 + ks + 1) * 64 + lane];
-#pragma unroll
-          for (int v = 0; v < 2; ++v) acc[v] = mfma32(a[v], bx[ks], acc[v]);
-          if ((ks & 1) && pending) store_pending(grp ? stage : stage - 1, grp ^ 1, ks >> 1);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int v = 0; v < 2; ++v)
-            if (ks + 1 < 16) a[v] = an[v];
-        }
-        if (stage < 8) {  // q (stages 0-3) or k (4-7): rotate interleaved pairs in fp32, pack bf16 rows
-          // q leaves in units of log2(e) (scores become base-2 exponents for the softmax); k as is
-          const float sc = stage < 4 ? kLog2e : 1.0f;
-#pragma unroll
-          for (int v = 0; v < 2; ++v) {
-            const int half = v;  // tiles 2grp and 2grp+1 are halves 0 and 1 of one head
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const float2 c = rc[half][g], sn = rsn[half][g];
-              const float a0 = acc[v][4 * g], a1 = acc[v][4 * g + 1], a2 = acc[v][4 * g + 2], a3 = acc[v][4 * g + 3];
-              u32x2 o = {0u, 0u};
-              if (valid) {
-                o[0] = pk_bf16(fmaf(a0, c.x, -(a1 * sn.x)) * sc, fmaf(a1, c.x, a0 * sn.x) * sc);
-                o[1] = pk_bf16(fmaf(a2, c.y, -(a3 * sn.y)) * sc, fmaf(a3, c.y, a2 * sn.y) * sc);
-              }
-              pend[4 * v + g] = o;
-            }
-          }
-        } else {  // v: register group g holds rows 8g + 4hh + r (r = 0..3) of position p; a 4 x 4
-          // transpose across each lane quad (two DPP exchanges) leaves lane 4q + r with row r of
-          // positions 4q..4q+3, so a half-wave's store covers 4 rows x 64 contiguous bytes.
-          const bool b1 = qd & 2, b0 = qd & 1;
-          // byte selectors of v_perm_b32 (bytes 0-3 from the second operand, 4-7 from the first)
-          const uint32_t sel_send = b0 ? 0x05040100u : 0x07060302u;
-          const uint32_t sel_f0 = b0 ? 0x03020504u : 0x05040100u;
-          const uint32_t sel_f1 = b0 ? 0x03020706u : 0x07060100u;
-#pragma unroll
-          for (int v = 0; v < 2; ++v)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              // d0/d1: rows (0,1)/(2,3) of this position (zero past the sequence end)
-              const uint32_t d0 = valid ? pk_bf16(acc[v][4 * g], acc[v][4 * g + 1]) : 0u;
-              const uint32_t d1 = valid ? pk_bf16(acc[v][4 * g + 2], acc[v][4 * g + 3]) : 0u;
-              // exchange with lane ^ 2: lanes 0,1 keep rows 0,1 of positions q, q+2; lanes 2,3 rows 2,3
-              const uint32_t r1 = uint32_t(__builtin_amdgcn_update_dpp(0, int(b1 ? d0 : d1), 0x4E, 0xF, 0xF, true));
-              const uint32_t e0 = b1 ? r1 : d0, e1 = b1 ? d1 : r1;
-              // exchange halves with lane ^ 1: lane r ends with row r of positions 0..3
-              const uint32_t snd = __builtin_amdgcn_perm(e1, e0, sel_send);
-              const uint32_t r2 = uint32_t(__builtin_amdgcn_update_dpp(0, int(snd), 0xB1, 0xF, 0xF, true));
-              pend[4 * v + g] = u32x2{__builtin_amdgcn_perm(r2, e0, sel_f0), __builtin_amdgcn_perm(r2, e1, sel_f1)};
-            }
-        }
+        for (int q = 0; q < 2; ++q)
+          __builtin_amdgcn_raw_buffer_store_b128(join_halves(o[2 * q], o[2 * q + 1]), res,
+                                                 ((4 * half + 2 * q + hh) * Lpad + p0 + 32 * ct + j) * 16, 0, 0);
       }
     }
-    // a block left before its gate stage: its last group's outputs leave now
-    if (active && st1 < kQkvStages) {
+  }
+  u32x2 vp[2][C][4];  // V^T: feature 32 half + j, positions 32 ct + 8g + 4hh + r
 #pragma unroll
-      for (int i = 0; i < kQkvGroupStores; ++i) store_pending(st1 - 1, 1, i);
-    }
+  for (int half = 0; half < 2; ++half) {
+    f32x16 acc[C];
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
+    tile_gemm<16, C, kFfBf16, 1, true>(w, tile(2, half).v, tile(2, 1).v, a, acc, xop, none);
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = p0 + 32 * ct + row_of_group(g, hh) + r < L ? acc[ct][4 * g + r] : 0.f;
+        vp[half][ct][g] = u32x2{pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3])};
+      }
+  }
+  lds_barrier();  // every wave has read the xn blocks and cos / sin rows
+  constexpr int CH = 4 * C, RI = 64 / CH;  // 16-byte chunks of a V^T row, rows of one store instruction
+  u32x4* const vs = smem + wave * (kHeadDim * CH);
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+#pragma unroll
+    for (int ct = 0; ct < C; ++ct)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = 32 * half + j;
+        reinterpret_cast<u32x2*>(vs)[2 * (d * CH + ((4 * ct + g) ^ (d & (CH - 1)))) + hh] = vp[half][ct][g];
+      }
+  const auto vres = buffer_rsrc(Vt + head0, kHeadDim * Lpad * 2);
+#pragma unroll
+  for (int i = 0; i < kHeadDim / RI; ++i) {
+    const int d = RI * i + lane / CH, c = lane & (CH - 1);
+    __builtin_amdgcn_raw_buffer_store_b128(vs[d * CH + (c ^ (d & (CH - 1)))], vres, (d * Lpad + p0) * 2 + c * 16, 0, 0);
   }
 }
 
@@ -356,21 +263,17 @@ int device_cu_count() {
   return n;
 }
 
-// Workgroups of the QKV kernel: one per CU (the kernel deals its units itself), at most one per unit.
-static int qkv_grid(int units) {
-  const int n = device_cu_count();
-  return units < n ? units : n;
-}
+// Token tiles of a launch over n rows: 32 rows while such tiles fit one per CU, 64 beyond.
+static int token_tiles(int64_t n) { return n <= int64_t(32) * device_cu_count() ? 1 : 2; }
 
 void launch_qkv(const uint16_t* xn, const uint8_t* layer, const float* rope, const SeqShape& sh, uint16_t* Q,
                 uint16_t* K, uint16_t* Vt, float* G, hipStream_t st, const LaunchEvents& ev) {
   const int64_t rows = int64_t(sh.nseq) * sh.Lpad;
-  const int nblocks = int((rows / 32 + kQkvWaves - 1) / kQkvWaves);
-  if (nblocks <= 0) return;
-  hipExtLaunchKernelGGL(k_qkv_rope, dim3(unsigned(qkv_grid(nblocks * kQkvStages))), dim3(64 * kQkvWaves), 0, st,
-                        ev.start, ev.stop, 0, xn, reinterpret_cast<const u32x4*>(layer + kOffQkvg),
-                        reinterpret_cast<const float*>(layer + kOffBgate), rope, sh.mode, sh.nseq, sh.L, sh.Lpad,
-                        sh.T, sh.F, nblocks, Q, K, Vt, G);
+  if (rows <= 0) return;
+  const int C = token_tiles(rows);
+  const auto kernel = C == 1 ? k_qkv_rope<1> : k_qkv_rope<2>;
+  hipExtLaunchKernelGGL(kernel, dim3(unsigned(rows / (32 * C))), dim3(64 * kTileWaves), 0, st, ev.start, ev.stop, 0,
+                        xn, layer, rope, sh.mode, sh.L, sh.Lpad, sh.T, sh.F, Q, K, Vt, G);
 }
 
 
@@ -858,52 +761,8 @@ __device__ __forceinline__ float gelu_logistic(float x) {
 }
 
 // ============================================================ token-tile GEMM kernels
-// The kernels from here on give a workgroup a tile of 32 C tokens (C = 1 or 2) and all output features:
-// its 8 waves split the features (32-row weight tiles), and the tile's activations sit in LDS, where
-// every wave reads them as B operands.  A wave's weight tiles are its own, so they go from L2 straight
-// into registers as A operands, kWeightAhead k-steps ahead of their MFMAs: nothing waits at a barrier for
-// weights, and one 1 KB block feeds C MFMAs.  What C and the register budget are chosen for: two
-// workgroups of 8 waves per CU (at most 128 VGPRs and 80 KB of LDS each), so that one's memory phases and
-// barriers run beside the other's matrix work.  The L2 delivers ~50 bytes per cycle per CU, which bounds
-// C = 1 (1.3 MB of a sub-layer's weights per 32 tokens); C = 4 fills a CU with one workgroup.  Full
-// post-attention block, us at C = 1 / 2 / 4: 18 / 24 / 45 at 6,262 tokens, 37 / 35 / 53 at 16,384,
-// 223 / 172 / 225 at 105,462.  So a launch takes C = 1 while its 32-token tiles fit one per CU and
-// C = 2 beyond.
-//
-// Rows of X, O, xn and H move in whole rows or half rows per wave instruction and are transposed through
-// LDS.  Loaded or stored in operand layout (32 rows x 16 bytes, the halves of a pair 32 lanes apart) an
-// instruction occupies the CU's address path several times as long: the out-projection, residual and
-// norm alone took 89 us at 105,462 tokens that way, 72 us through LDS (378 MB: the HBM rate of a copy).
-// 1 KB rows are held as 64 16-byte chunks, chunk c of token t at c ^ (t & 15): the 16 lanes of an LDS
-// access then touch 16 different chunks of their 256 bytes.
-constexpr int kTileWaves = 8;
-constexpr int kWeightAhead = 4;  // k-steps a wave's weight blocks are loaded ahead (8 spills at C = 2)
+// Workgroups of 8 waves on tiles of 32 C tokens, see trf_tiles.h.
 constexpr int kDropOffset = 0x7ffffff0;  // a buffer offset past every resource: its loads give zeros
-
-inline int token_tiles(int64_t n) { return n <= int64_t(32) * device_cu_count() ? 1 : 2; }
-
-__device__ __forceinline__ u32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
-
-// This wave's LDS operations have completed, then all waves meet; its global loads stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // vmcnt(63) expcnt(7) lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Everything this wave loads (direct-to-LDS loads too) has landed, then all waves meet.
-__device__ __forceinline__ void loads_barrier() {
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) expcnt(7) lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Position of chunk c of token t in a tile of 1 KB rows.
-__device__ __forceinline__ int row_chunk(int t, int c) { return t * 64 + (c ^ (t & 15)); }
 
 // The norms of a tile's tokens: wave w's partial sum of squares of token t is ssq[t * kTileWaves + w].
 template <int C>
@@ -1200,17 +1059,11 @@ void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* 
 // overlap only in part (priorities for one of a CU's two workgroups change nothing).
 // (fast.py:311-331, kernels.cpp:542-642)
 
-// FF operand packing and products of the one-part arithmetics.
+// FF operand packing of the one-part arithmetics.
 template <int PREC>
 __device__ __forceinline__ uint32_t pk_ff(float lo, float hi) {
   return PREC == kFfFp16 ? pk_f16(lo, hi) : pk_bf16(lo, hi);
 }
-template <int PREC>
-__device__ __forceinline__ f32x16 mfma_ff(u32x4 a, u32x4 b, f32x16 c) {
-  return PREC == kFfFp16 ? mfma32h(a, b, c) : mfma32(a, b, c);
-}
-__host__ __device__ constexpr int ff_parts(int prec) { return prec == kFfSplit ? 2 : 1; }
-
 // The bf16 hi and lo parts of a pair.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
   hi = pk_bf16(a, b);
@@ -1228,62 +1081,6 @@ __device__ __forceinline__ void pack_ff(float a, float b, u32x4 (&v)[ff_parts(PR
   } else {
     v[0][q] = pk_ff<PREC>(a, b);
   }
-}
-
-// A wave's stream of weight blocks: k-step k of the current GEMM is at off[part] + k KB of the layer.
-struct PaWeights {
-  __amdgpu_buffer_rsrc_t res;
-  int lane16;
-  __device__ __forceinline__ u32x4 load(int off) const { return buffer_load16(res, lane16, off); }
-};
-
-// acc += W . B over KS k-steps.  a holds the first kWeightAhead k-steps' blocks and is left with those of
-// the next GEMM (at next[], NEXT parts; 0: there is none).  b(k, part, ct) is the LDS operand.  side(k) is
-// VALU work placed beside k-step k's MFMAs.
-template <int KS, int C, int PREC, int NEXT, typename Operand, typename Side>
-__device__ __forceinline__ void pa_gemm(const PaWeights& w, const int (&off)[2], const int (&next)[2],
-                                        u32x4 (&a)[kWeightAhead][2], f32x16 (&acc)[C], Operand&& operand,
-                                        Side&& side) {
-  constexpr int NP = ff_parts(PREC);
-  constexpr int AHEAD = C == 1 ? (NP == 1 ? 4 : 2) : 1;  // k-steps the activation operands are read ahead
-  u32x4 b[AHEAD + 1][NP][C];
-  auto read = [&](int k) __attribute__((always_inline)) {
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-      for (int ct = 0; ct < C; ++ct) b[k % (AHEAD + 1)][p][ct] = operand(k, p, ct);
-  };
-#pragma unroll
-  for (int k = 0; k < AHEAD; ++k) read(k);
-#pragma unroll
-  for (int k = 0; k < KS; ++k) {
-    if (k + AHEAD < KS) read(k + AHEAD);
-    __builtin_amdgcn_sched_barrier(0);
-    u32x4 (&ak)[2] = a[k % kWeightAhead];
-    u32x4 (&bk)[NP][C] = b[k % (AHEAD + 1)];
-#pragma unroll
-    for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[0], bk[0][ct], acc[ct]);
-    if constexpr (NP == 2) {
-#pragma unroll
-      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[0], bk[1][ct], acc[ct]);
-#pragma unroll
-      for (int ct = 0; ct < C; ++ct) acc[ct] = mfma_ff<PREC>(ak[1], bk[0][ct], acc[ct]);
-    }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      if (k + kWeightAhead < KS) {
-        if (p < NP) ak[p] = w.load(off[p] + (k + kWeightAhead) * kTileBytes);
-      } else if (p < NEXT) {
-        ak[p] = w.load(next[p] + (k + kWeightAhead - KS) * kTileBytes);
-      }
-    }
-    side(k);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // The products end here: without this the compiler may sink the whole MFMA chain, whose only readers come
-  // later, past the next barrier, and keep every operand in scratch until then.
-#pragma unroll
-  for (int ct = 0; ct < C; ++ct) asm volatile("" : "+v"(acc[ct]));
 }
 
 // The split arithmetic at C = 2 holds 128 KB of operands: one workgroup per CU, 256 registers a wave.
@@ -1308,7 +1105,7 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
   const int rows = int(n - tok0 < R ? n - tok0 : R);  // rows past the last token read as zeros, stores drop
   const auto xres = buffer_rsrc(X + tok0 * kDim, rows * kDim * 4);
   const auto nres = buffer_rsrc(xn + tok0 * kDim, xn ? rows * kDim * 2 : 0);
-  const PaWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
+  const TileWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
   {
     static_assert(kDim * 4 == 512 * 2, "rows of O and X are 1 KB");
     const auto rres = OUTPROJ ? buffer_rsrc(O + tok0 * 512, rows * 1024) : xres;
@@ -1325,15 +1122,12 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
   }
   constexpr int w1[2] = {int(PREC == kFfFp16 ? kOffFf1F16 : kOffFf1), int(kOffFf1Lo)};
   constexpr int w2[2] = {int(PREC == kFfFp16 ? kOffFf2F16 : kOffFf2), int(kOffFf2Lo)};
-  struct Off {
-    int v[2];
-  };
-  const Off out{{int(kOffOut) + wave * 32 * kTileBytes, 0}};
-  auto ff1 = [&](int c) __attribute__((always_inline)) { return Off{{w1[0] + (8 * c + wave) * 16 * kTileBytes, w1[1] + (8 * c + wave) * 16 * kTileBytes}}; };
-  auto ff2 = [&](int c) __attribute__((always_inline)) { return Off{{w2[0] + (64 * wave + 16 * c) * kTileBytes, w2[1] + (64 * wave + 16 * c) * kTileBytes}}; };
+  const TileOff out{{int(kOffOut) + wave * 32 * kTileBytes, 0}};
+  auto ff1 = [&](int c) __attribute__((always_inline)) { return TileOff{{w1[0] + (8 * c + wave) * 16 * kTileBytes, w1[1] + (8 * c + wave) * 16 * kTileBytes}}; };
+  auto ff2 = [&](int c) __attribute__((always_inline)) { return TileOff{{w2[0] + (64 * wave + 16 * c) * kTileBytes, w2[1] + (64 * wave + 16 * c) * kTileBytes}}; };
   u32x4 a[kWeightAhead][2];
   {
-    const Off first = OUTPROJ ? out : ff1(0);
+    const TileOff first = OUTPROJ ? out : ff1(0);
 #pragma unroll
     for (int i = 0; i < kWeightAhead; ++i)
 #pragma unroll
@@ -1346,7 +1140,7 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
 #pragma unroll
     for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
     const int m = j & 15, base = j * 64 + (hh ^ (m & 1)), me = m & 14;  // chunk 2k + hh of token j
-    pa_gemm<32, C, kFfBf16, NP>(w, out.v, ff1(0).v, a, acc,
+    tile_gemm<32, C, kFfBf16, NP>(w, out.v, ff1(0).v, a, acc,
                                 [&](int k, int, int ct) __attribute__((always_inline)) {
                                   return smem[base + ((2 * k) ^ me) + ct * 32 * 64];
                                 },
@@ -1414,15 +1208,15 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
   auto hop = [&](int k, int p, int ct) __attribute__((always_inline)) { return hb[p * kPart + (ct * 16 + k) * 64 + lane]; };
   constexpr int kBlocks = kHidden / 256;
   start_h(0);
-  pa_gemm<16, C, PREC, NP>(w, ff1(0).v, ff1(1).v, a, h, xop, none);
+  tile_gemm<16, C, PREC, NP>(w, ff1(0).v, ff1(1).v, a, h, xop, none);
 #pragma unroll
   for (int v = 0; v < 8 * C; ++v) gelu_pair(v);
   put_h();
 #pragma unroll
   for (int c = 1; c < kBlocks; ++c) {
     start_h(c);
-    pa_gemm<16, C, PREC, NP>(w, ff1(c).v, ff2(c - 1).v, a, h, xop, none);
-    pa_gemm<16, C, PREC, NP>(w, ff2(c - 1).v, (c + 1 < kBlocks ? ff1(c + 1) : ff2(c)).v, a, acc, hop,
+    tile_gemm<16, C, PREC, NP>(w, ff1(c).v, ff2(c - 1).v, a, h, xop, none);
+    tile_gemm<16, C, PREC, NP>(w, ff2(c - 1).v, (c + 1 < kBlocks ? ff1(c + 1) : ff2(c)).v, a, acc, hop,
                              [&](int k) __attribute__((always_inline)) {
 #pragma unroll
                                for (int v = k * C / 2; v < (k + 1) * C / 2; ++v) gelu_pair(v);
@@ -1430,7 +1224,7 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
     lds_barrier();  // every wave has read block c - 1
     put_h();
   }
-  pa_gemm<16, C, PREC, 0>(w, ff2(kBlocks - 1).v, out.v, a, acc, hop, none);
+  tile_gemm<16, C, PREC, 0>(w, ff2(kBlocks - 1).v, out.v, a, acc, hop, none);
   put_ssq(acc, ssq, wave, j, hh);
   lds_barrier();
   store_tile(acc, smem, ssq, eps, xres, nres, wave, lane);
