@@ -5,456 +5,187 @@
 // bf16 rounding, bf16 q, k, v and unnormalised P, the exact row max over the valid keys, an fp32 sum of
 // e = 2^(s - m), and O = (P.V) * gate / sum rounded to bf16 in token order.
 //
-// A sequence is two 32-position halves, one wave each, and the two waves of a sequence share a SIMD, so
-// each SIMD runs two waves and one wave's rotary, softmax and packing work can run under the other's
-// MFMAs.  A wave keeps its 32 positions' xn rows in registers (bf16, natural k order) and computes q, k
-// and v of its own positions; each half writes its K and V^T operand blocks to LDS and reads the other
-// half's, so that every wave attends its 32 queries over all 64 keys.  A workgroup is 4 sequences (8
-// waves).  The 49 weight tiles of W_qkvg stream through LDS: the gate tile, then per head stage A (the q
-// and k tiles, 64 KB) and stage B (the v tiles, 32 KB), each in its own buffer so that one loads while the
-// other is read (160 KB of LDS with the exchange blocks).
-//
-// Work is dealt in units of (group of 4 sequences, head): workgroup b of G runs units [bU/G, (b+1)U/G)
-// of the U = 8 x groups in order, so one workgroup per CU gets an even share of heads (13 or 14 units
-// for the 1701 frames of a 17 s chunk) instead of two rounds of whole groups (1.66 groups per CU).  A
-// group entered mid-way or left early loads its xn rows and computes its gates again.
-//
-// Per head h:
-//   A: P.V of head h - 1 (its V^T now visible from both halves) and its 8 bounds-checked O stores,
-//      spread between the q products of head h; then the k products with the rotary of q between them;
-//      then the rotary of k, written to LDS;
-//   B: S^T = K.Q^T over both halves' keys, then the v products with the softmax of S^T between them;
-//      then V^T packed and written to LDS.
-// The stage barriers wait for the stage's loads with an exact vmcnt (the 8 O stores of a head are
-// issued after the loads of stage B and are never waited for) and for the LDS exchange.
+// A workgroup is 4 heads of one sequence after another, padded to 32 C positions (C = 1 up to 32 positions,
+// else 2), and a wave is one head from its projections to its output (trf_tiles.h has the staging and the
+// weight streaming).  The waves meet twice per sequence, when its xn rows are in LDS and before the next
+// one's replace them; in between each runs on its own, so that one wave's rotary, softmax and packing run
+// under another's MFMAs.  The next sequence's xn is loaded during the attention.  At C = 2 a wave holds the q,
+// k and v operands of 64 positions (96 registers): two workgroups a CU, two waves a SIMD.
 //
 // No data crosses lanes between the projection and the attention:
 //   * q and k come out of C = W . xn^T with lane (j, hh) holding token j of the column tile and features
 //     8g + 4hh + r.  Packed to bf16 in that "register order", q is the B operand (Q^T) and k the A
 //     operand (K) of S^T = K . Q^T: both use the same permutation of the 16 head features of a k-step,
 //     which leaves the dot products unchanged.
-//   * v comes out of the swapped product C = xn . W_v^T (the xn registers are the A operand, the packed
-//     W_v block the B operand), so lane (j, hh) holds feature j of tokens 8g + 4hh + r: exactly the
-//     A operand (V^T) of O^T = V^T . P^T with the keys of a k-step in the register order in which the
-//     S^T accumulator holds them, so P^T is the B operand straight from the accumulator.
+//   * v comes out of the swapped product C = xn . W_v^T (the xn rows are the A operand, the packed W_v
+//     block the B operand), so lane (j, hh) holds feature j of tokens 8g + 4hh + r: exactly the A operand
+//     (V^T) of O^T = V^T . P^T with the keys of a k-step in the register order in which the S^T accumulator
+//     holds them, so P^T is the B operand straight from the accumulator.
 // The row max and the row sum combine the two half-waves (the query's keys sit in lanes j and j + 32).
-#include "trf_device.h"
+// O leaves through the wave's own LDS rows as whole 128-byte lines.
+//
+// Against workgroups of 4 sequences that streamed the weights through LDS and exchanged K and V^T between
+// position halves (us): 62 positions, 251 sequences 35 and 23; 101 sequences 19.5 and 17; 1701 the same within 1%.  At 1701 the
+// MFMA pipe is busy 40%, the address units 46%, LDS 36% of the time; 8 weight k-steps ahead instead of 4, and
+// 8 heads a workgroup instead of 4, changed nothing there.
+#include "trf_tiles.h"
 
 namespace trf {
 
-constexpr int kFsSeqs = 4;                       // sequences per workgroup
-constexpr int kFsWaves = 2 * kFsSeqs;            // one wave per 32-position half; waves w, w + 4 share a SIMD
-constexpr int kFsBlocksA = 64;                   // q and k tiles of a head: 2 kinds x 2 halves x 16 k-steps
-constexpr int kFsBlocksB = 32;                   // v tiles of a head: 2 halves x 16 k-steps
-constexpr int kFsBlocksG = 16;                   // the gate tile (in stage B's buffer)
-constexpr int kFsStoresPerHead = 8;              // O stores per wave and head: 2 feature tiles x 4 groups
-// LDS layout, in 16-byte units: stage A, stage B, then the K and V^T operand blocks exchanged between
-// the halves, [sequence][half][k-step][lane] (160 KB).
-constexpr int kFsOffB = kFsBlocksA * 64;
-constexpr int kFsOffKx = kFsOffB + kFsBlocksB * 64;
-constexpr int kFsOffVx = kFsOffKx + kFsSeqs * 2 * 4 * 64;
-constexpr int kFsLdsVecs = kFsOffVx + kFsSeqs * 2 * 4 * 64;
 constexpr int kFsDropped = kFusedShortDropped;  // buffer offset past any sequence's output: the store is dropped
-
-// This wave's share of the gate tile (the last tile of W_qkvg).
-__device__ __forceinline__ void fs_issue_gate(u32x4* buf, const u32x4* wq, int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < kFsBlocksG / kFsWaves; ++i) {
-    const int b = (kFsBlocksG / kFsWaves) * wave + i;
-    lds_load_block(wq + (int64_t(kQkvgTiles - 1) * 16 + b) * 64, buf + b * 64, lane);
-  }
-}
-
-// Stage A of head h: block 32 kind + 16 c + ks is k-step ks of tile 16 kind + 2h + c (kind 0 q, 1 k).
-__device__ __forceinline__ void fs_issue_a(int h, u32x4* buf, const u32x4* wq, int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < kFsBlocksA / kFsWaves; ++i) {
-    const int b = (kFsBlocksA / kFsWaves) * wave + i;
-    const int t = 16 * (b >> 5) + 2 * h + ((b >> 4) & 1);
-    lds_load_block(wq + (int64_t(t) * 16 + (b & 15)) * 64, buf + b * 64, lane);
-  }
-}
-
-// Stage B of head h: block 16 c + ks is k-step ks of v tile 32 + 2h + c.
-__device__ __forceinline__ void fs_issue_b(int h, u32x4* buf, const u32x4* wq, int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < kFsBlocksB / kFsWaves; ++i) {
-    const int b = (kFsBlocksB / kFsWaves) * wave + i;
-    const int t = 32 + 2 * h + (b >> 4);
-    lds_load_block(wq + (int64_t(t) * 16 + (b & 15)) * 64, buf + b * 64, lane);
-  }
-}
-
-// This thread's vector memory operations have completed except the N most recent, its LDS operations
-// have all completed (the K / V^T exchange), then all waves meet.
-template <int N>
-__device__ __forceinline__ void fs_barrier() {
-  static_assert(N >= 0 && N < 64, "vmcnt field");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0070);  // vmcnt(N) expcnt(7) lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // Key (or token) of register R of half-wave hh in a 32-row accumulator tile: row 8(R/4) + 4hh + R%4.
 __device__ __forceinline__ int acc_row(int R, int hh) { return 8 * (R >> 2) + 4 * hh + (R & 3); }
 
-// The rotary cos/sin of this lane's position: pairs 16c + 4g + 2hh + {0, 1}, the ones that register
-// group g (rows 8g + 4hh + r) of head half c rotates.
-struct FsRope {
-  float2 cs[2][4], sn[2][4];
-};
-
-// Rotary of register group g of head half c, fp32, scaled, into the bf16 operand of k-step 2c + g/2
-// (elements 2(g%2), 2(g%2) + 1).
-__device__ __forceinline__ void fs_rotate(const f32x16& a, const FsRope& rp, int c, int g, float scale, u32x4& out) {
-  const float2 cs = rp.cs[c][g], sn = rp.sn[c][g];
-  const float a0 = a[4 * g], a1 = a[4 * g + 1], a2 = a[4 * g + 2], a3 = a[4 * g + 3];
-  out[2 * (g & 1)] = pk_bf16(fmaf(a0, cs.x, -(a1 * sn.x)) * scale, fmaf(a1, cs.x, a0 * sn.x) * scale);
-  out[2 * (g & 1) + 1] = pk_bf16(fmaf(a2, cs.y, -(a3 * sn.y)) * scale, fmaf(a3, cs.y, a2 * sn.y) * scale);
+// Two k-steps' operands from a tile's accumulators, in register order.
+__device__ __forceinline__ void pack_tile(const f32x16& v, u32x4 (&out)[2]) {
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+    out[kk] = u32x4{pk_bf16(v[8 * kk], v[8 * kk + 1]), pk_bf16(v[8 * kk + 2], v[8 * kk + 3]),
+                    pk_bf16(v[8 * kk + 4], v[8 * kk + 5]), pk_bf16(v[8 * kk + 6], v[8 * kk + 7])};
 }
 
-// One head's output of this wave's 32 queries, from P.V to the store: O^T accumulators [feature tile],
-// the per-query scale gate / sum and the query row's byte offset (kFsDropped past the sequence end).
-struct FsOut {
-  f32x16 o[2];
-  float sc;
-  int off;
-};
+// The operands are formed here, before the next tile's products: left to itself the compiler forms them where
+// they are read, and keeps the fp32 tiles until then.
+__device__ __forceinline__ void pin(u32x4 (&v)[2]) { asm volatile("" : "+v"(v[0]), "+v"(v[1])::"memory"); }
 
-// Store unit u (0..7) of a head's output: feature tile u / 4, register group u % 4.
-__device__ __forceinline__ void fs_store_unit(const FsOut& po, int u, int h, int hh, __amdgpu_buffer_rsrc_t ores) {
-  const int dt = u >> 2, g = u & 3;
-  const f32x16& o = po.o[dt];
-  const u32x2 v = {pk_bf16(o[4 * g] * po.sc, o[4 * g + 1] * po.sc), pk_bf16(o[4 * g + 2] * po.sc, o[4 * g + 3] * po.sc)};
-  const int off = po.off + 2 * (h * kHeadDim + 32 * dt + row_of_group(g, hh));
-  __builtin_amdgcn_raw_buffer_store_b64(v, ores, off, 0, 0);
-}
+constexpr int kFsWaves = 4;  // one head each
 
-// What one head leaves for the next head's stage A: this half's V^T operands [feature tile][key k-step], the
-// P^T operands of its queries [key k-step 2 kt + kk], and the scale and offset of its output.
-struct FsCarry {
-  u32x4 vb[2][2];
-  u32x4 pb[4];
-  float sc;
-  int off;
-};
-
-// P.V of a head: the other half's V^T operands come from LDS.
-__device__ __forceinline__ void fs_pv(const FsCarry& cy, const u32x4* __restrict__ vx_other, int th, int lane,
-                                      FsOut& po) {
+template <int C>
+__global__ __launch_bounds__(64 * kFsWaves, 2) void k_qkv_attn_short(
+    const uint16_t* __restrict__ xn, const uint8_t* __restrict__ layer, const float* __restrict__ rope, int mode,
+    int nseq, int L, int T, int F, uint16_t* __restrict__ O) {
+  constexpr int R = 32 * C;
+  constexpr int kRope = R * 32, kGate = kRope + R * kRopeChunks, kOut = kGate + kFsWaves * R * kHeads / 4;
+  __shared__ u32x4 smem[kOut + kFsWaves * 32 * 8];  // xn, cos | sin, partial gates, 32 output rows a wave
+  float* const gates = reinterpret_cast<float*>(smem + kGate);
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int j = lane & 31, hh = lane >> 5, h = kFsWaves * (blockIdx.x & 1) + wave;
+  const TileWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
+  auto tile = [&](int kind, int half) __attribute__((always_inline)) {  // kind 0 q, 1 k, 2 v
+    return TileOff{{int(kOffQkvg) + (16 * kind + 2 * h + half) * 16 * kTileBytes, 0}};
+  };
+  auto xop = [&](int k, int, int ct) __attribute__((always_inline)) { return smem[(ct * 16 + k) * 64 + lane]; };
+  auto none = [](int) __attribute__((always_inline)) {};
+  const int stride = mode == 0 ? F : 1;  // tokens between positions
+  u32x4* const os = smem + kOut + wave * 32 * 8;
+  TilePositions<C, kFsWaves> x;
+  x.load(xn, mode, blockIdx.x >> 1, 0, L, T, F);
+  u32x4 a[kWeightAhead][2], ag[16 / kFsWaves];
 #pragma unroll
-  for (int dt = 0; dt < 2; ++dt) {
-    po.o[dt] = zero16();
+  for (int i = 0; i < 16 / kFsWaves; ++i)
+    ag[i] = w.load(int(kOffQkvg) + ((kQkvgTiles - 1) * 16 + 16 / kFsWaves * wave + i) * kTileBytes);
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+  for (int i = 0; i < kWeightAhead; ++i) a[i][0] = w.load(tile(2, 0).v[0] + i * kTileBytes);
+  stage_rope<C, kFsWaves>(rope, 0, L, smem + kRope);
+#pragma unroll 1
+  for (int s = blockIdx.x >> 1; s < nseq; s += gridDim.x >> 1) {
+    x.put(smem);
+    lds_barrier();
+    gate_partials<C, kFsWaves>(ag, smem, gates, wave, lane);
+    u32x4 vb[2][C][2], kb[2][C][2], qb[2][C][2];  // [head half][position tile][k-step]
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const u32x4 v = kt == th ? cy.vb[dt][kk] : vx_other[(2 * dt + kk) * 64 + lane];
-        po.o[dt] = mfma32(v, cy.pb[2 * kt + kk], po.o[dt]);
-      }
-  }
-  po.sc = cy.sc;
-  po.off = cy.off;
-}
-
-struct FsCtx {
-  const u32x4* wq;
-  FsRope rope;
-  const u32x4* kx_other;
-  u32x4* kx_own;
-  const u32x4* vx_other;
-  u32x4* vx_own;
-  __amdgpu_buffer_rsrc_t ores;
-  int qoff, L, p, th, hh, lane, wave;
-  bool active;
-  float gv[4];  // sigmoid gates of heads 4hh + r for this lane's query
-};
-
-// One head: stage A (q and k) and stage B (v, attention).  hn is the head of the workgroup's next unit
-// (its stage A is loaded during stage B), or -1.  CARRY: the previous head of the same group was run
-// here, and its P.V and stores happen in this head's stage A.
-template <bool CARRY>
-__device__ __forceinline__ void fs_head(int h, int hn, const FsCtx& cx, u32x4* smem, const u32x4 (&bx)[16],
-                                        FsCarry& cy) {
-  u32x4* const La = smem;
-  u32x4* const Lb = smem + kFsOffB;
-  const int lane = cx.lane;
-
-  // ---- stage A: P.V and stores of head h - 1 between the q products of head h, then the k products
-  // with the rotary of q between them, then the rotary of k into LDS
-  fs_barrier<0>();  // stage A landed; V^T of head h - 1 written by both halves
-  fs_issue_b(h, Lb, cx.wq, cx.wave, lane);
-  u32x4 qb[2][2], kb[2][2];  // [head half][k-step of the half]
-  if (cx.active) {
-    f32x16 qa[2];
-    {
-      FsOut po;
-      if (CARRY) fs_pv(cy, cx.vx_other, cx.th, lane, po);
+    for (int i = 0; i < 6; ++i) {  // the v, k and q tiles; the last one's next is the next sequence's first
+      const int kind = 2 - i / 2, half = i & 1;
+      const TileOff off = tile(kind, half), next = i == 5 ? tile(2, 0) : half ? tile(kind - 1, 0) : tile(kind, 1);
+      f32x16 acc[C];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) qa[c] = zero16();
-      u32x4 a0 = La[lane], a1 = La[16 * 64 + lane];
+      for (int ct = 0; ct < C; ++ct) acc[ct] = zero16();
+      if (kind == 2)
+        tile_gemm<16, C, kFfBf16, 1, true, 1>(w, off.v, next.v, a, acc, xop, none);
+      else
+        tile_gemm<16, C, kFfBf16, 1, false, 1>(w, off.v, next.v, a, acc, xop, none);
 #pragma unroll
-      for (int ks = 0; ks < 16; ++ks) {
-        u32x4 n0, n1;
-        if (ks + 1 < 16) {
-          n0 = La[(ks + 1) * 64 + lane];
-          n1 = La[(16 + ks + 1) * 64 + lane];
+      for (int ct = 0; ct < C; ++ct) {
+        if (kind == 2) {
+          pack_tile(acc[ct], vb[half][ct]);
+          pin(vb[half][ct]);
+          continue;
         }
-        qa[0] = mfma32(a0, bx[ks], qa[0]);
-        qa[1] = mfma32(a1, bx[ks], qa[1]);
-        if (CARRY && (ks & 1)) fs_store_unit(po, ks >> 1, h - 1, cx.hh, cx.ores);
-        __builtin_amdgcn_sched_barrier(0);
-        if (ks + 1 < 16) {
-          a0 = n0;
-          a1 = n1;
+        u32x4 (&out)[2] = kind == 1 ? kb[half][ct] : qb[half][ct];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const u32x2 o = rotate_group(acc[ct], g, smem + kRope, 32 * ct + j, half, hh, kind == 1 ? 1.0f : kLog2e);
+          out[g >> 1][2 * (g & 1)] = o[0];
+          out[g >> 1][2 * (g & 1) + 1] = o[1];
         }
+        pin(out);
       }
     }
-    f32x16 ka[2];
+    lds_barrier();  // the partial gates are there, and every wave has read xn
+    if (s + int(gridDim.x >> 1) < nseq) x.load(xn, mode, s + (gridDim.x >> 1), 0, L, T, F);
+    const auto ores = buffer_rsrc(O + token_of(mode, s, 0, T, F) * (kHeads * kHeadDim),
+                                  ((L - 1) * stride + 1) * kHeads * kHeadDim * 2);
 #pragma unroll
-    for (int c = 0; c < 2; ++c) ka[c] = zero16();
-    const u32x4* const Lk = La + 32 * 64;
-    u32x4 a0 = Lk[lane], a1 = Lk[16 * 64 + lane];
+    for (int qt = 0; qt < C; ++qt) {
+      f32x16 sacc[C];
 #pragma unroll
-    for (int ks = 0; ks < 16; ++ks) {
-      u32x4 n0, n1;
-      if (ks + 1 < 16) {
-        n0 = Lk[(ks + 1) * 64 + lane];
-        n1 = Lk[(16 + ks + 1) * 64 + lane];
+      for (int kt = 0; kt < C; ++kt) {
+        sacc[kt] = zero16();
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) sacc[kt] = mfma32(kb[half][kt][kk], qb[half][qt][kk], sacc[kt]);
       }
-      ka[0] = mfma32(a0, bx[ks], ka[0]);
-      ka[1] = mfma32(a1, bx[ks], ka[1]);
-      if (ks & 1) {
-        const int u = ks >> 1, c = u >> 2, g = u & 3;
-        fs_rotate(qa[c], cx.rope, c, g, kLog2e, qb[c][g >> 1]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if (ks + 1 < 16) {
-        a0 = n0;
-        a1 = n1;
-      }
-    }
+      float mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) fs_rotate(ka[u >> 2], cx.rope, u >> 2, u & 3, 1.0f, kb[u >> 2][(u & 3) >> 1]);
+      for (int kt = 0; kt < C; ++kt) {
+        if (32 * kt + 32 <= L) {  // a key tile with no padded keys (uniform): no masking
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) cx.kx_own[(2 * c + kk) * 64 + lane] = kb[c][kk];
-  }
-
-  // ---- stage B: S^T over both halves' keys, v products with the softmax between them, V^T into LDS
-  if (cx.active && CARRY)
-    fs_barrier<kFsStoresPerHead>();  // stage B landed (the 8 stores above are younger); K written
-  else
-    fs_barrier<0>();
-  if (hn >= 0) fs_issue_a(hn, La, cx.wq, cx.wave, lane);
-  if (cx.active) {
-    f32x16 sacc[2];  // [key tile]
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      sacc[kt] = zero16();
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const u32x4 k = kt == cx.th ? kb[c][kk] : cx.kx_other[(2 * c + kk) * 64 + lane];
-          sacc[kt] = mfma32(k, qb[c][kk], sacc[kt]);
-        }
-    }
-    f32x16 va[2];  // [head half]: features 32c + j of tokens 8g + 4hh + r
-#pragma unroll
-    for (int c = 0; c < 2; ++c) va[c] = zero16();
-    float m = 0.f, lsum = 0.f;
-    const int L = cx.L, hh = cx.hh;
-    u32x4 a0 = Lb[lane], a1 = Lb[16 * 64 + lane];
-#pragma unroll
-    for (int ks = 0; ks < 16; ++ks) {
-      u32x4 n0, n1;
-      if (ks + 1 < 16) {
-        n0 = Lb[(ks + 1) * 64 + lane];
-        n1 = Lb[(16 + ks + 1) * 64 + lane];
-      }
-      va[0] = mfma32(bx[ks], a0, va[0]);
-      va[1] = mfma32(bx[ks], a1, va[1]);
-      // softmax units after k-steps 1, 5, 9: the row max over the valid keys, then for each key tile
-      // e = 2^(s - m), its fp32 sum and the bf16 P^T operands
-      if (ks == 1) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-          if (32 * kt + 32 <= L) {  // a key tile with no padded keys (uniform): no masking
-#pragma unroll
-            for (int R = 0; R < 16; R += 2) mx = fmaxf(fmaxf(mx, sacc[kt][R]), sacc[kt][R + 1]);
-          } else {
-#pragma unroll
-            for (int R = 0; R < 16; ++R)
-              if (32 * kt + acc_row(R, hh) < L) mx = fmaxf(mx, sacc[kt][R]);
-          }
-        }
-        m = halfwave_max(mx);
-      } else if (ks == 5 || ks == 9) {
-        const int kt = ks == 5 ? 0 : 1;
-        float e[16];
-        if (32 * kt + 32 <= L) {
-#pragma unroll
-          for (int R = 0; R < 16; ++R) e[R] = __builtin_amdgcn_exp2f(sacc[kt][R] - m);
+          for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(mx, sacc[kt][r]), sacc[kt][r + 1]);
         } else {
 #pragma unroll
-          for (int R = 0; R < 16; ++R)
-            e[R] = 32 * kt + acc_row(R, hh) < L ? __builtin_amdgcn_exp2f(sacc[kt][R] - m) : 0.f;
+          for (int r = 0; r < 16; ++r)
+            if (32 * kt + acc_row(r, hh) < L) mx = fmaxf(mx, sacc[kt][r]);
         }
-#pragma unroll
-        for (int R = 0; R < 16; ++R) lsum += e[R];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-          cy.pb[2 * kt + kk] = u32x4{pk_bf16(e[8 * kk], e[8 * kk + 1]), pk_bf16(e[8 * kk + 2], e[8 * kk + 3]),
-                                     pk_bf16(e[8 * kk + 4], e[8 * kk + 5]), pk_bf16(e[8 * kk + 6], e[8 * kk + 7])};
       }
-      __builtin_amdgcn_sched_barrier(0);
-      if (ks + 1 < 16) {
-        a0 = n0;
-        a1 = n1;
+      const float m = halfwave_max(mx);
+      float lsum = 0.f;
+      f32x16 o[2] = {zero16(), zero16()};
+#pragma unroll
+      for (int kt = 0; kt < C; ++kt) {
+        f32x16 e;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const bool in = 32 * kt + 32 <= L || 32 * kt + acc_row(r, hh) < L;
+          e[r] = in ? __builtin_amdgcn_exp2f(sacc[kt][r] - m) : 0.f;
+          lsum += e[r];
+        }
+        u32x4 pb[2];
+        pack_tile(e, pb);
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) o[dt] = mfma32(vb[dt][kt][kk], pb[kk], o[dt]);
+      }
+      const float sc = gate_of<C, kFsWaves>(gates, 32 * qt + j, h, reinterpret_cast<const float*>(layer + kOffBgate)) *
+                       (1.0f / (lsum + __shfl_xor(lsum, 32)));
+      // rows of 8 chunks (the head's 64 features), chunk c of row t at c ^ (t & 7)
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          reinterpret_cast<u32x2*>(os)[2 * (j * 8 + ((4 * dt + g) ^ (j & 7))) + hh] =
+              u32x2{pk_bf16(o[dt][4 * g] * sc, o[dt][4 * g + 1] * sc),
+                    pk_bf16(o[dt][4 * g + 2] * sc, o[dt][4 * g + 3] * sc)};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 8 * i + (lane >> 3), c = lane & 7, p = 32 * qt + t;
+        const int off = p < L ? p * stride * (kHeads * kHeadDim * 2) + h * (kHeadDim * 2) + 16 * c : kFsDropped;
+        __builtin_amdgcn_raw_buffer_store_b128(os[t * 8 + (c ^ (t & 7))], ores, off, 0, 0);
       }
     }
-    // V^T operands of this half's keys [feature tile c][key k-step kk], kept and written to LDS
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
-        const f32x16& v = va[c];
-        cy.vb[c][kk] = u32x4{pk_bf16(v[8 * kk], v[8 * kk + 1]), pk_bf16(v[8 * kk + 2], v[8 * kk + 3]),
-                             pk_bf16(v[8 * kk + 4], v[8 * kk + 5]), pk_bf16(v[8 * kk + 6], v[8 * kk + 7])};
-        cx.vx_own[(2 * c + kk) * 64 + lane] = cy.vb[c][kk];
-      }
-    // gate of head h for this query: in this lane if h / 4 == hh, else in the partner lane
-    float own = cx.gv[0];
-#pragma unroll
-    for (int r = 1; r < 4; ++r) own = (h & 3) == r ? cx.gv[r] : own;
-    const float other = __shfl_xor(own, 32);
-    const float ls = lsum + __shfl_xor(lsum, 32);
-    cy.sc = (hh == (h >> 2) ? own : other) * (1.0f / ls);
-    cy.off = cx.qoff;
   }
-}
-
-// The last head's P.V and stores of a group, once both halves have written its V^T.
-__device__ __forceinline__ void fs_flush(const FsCtx& cx, const FsCarry& cy, int h) {
-  fs_barrier<0>();
-  if (cx.active) {
-    FsOut po;
-    fs_pv(cy, cx.vx_other, cx.th, cx.lane, po);
-#pragma unroll
-    for (int u = 0; u < kFsStoresPerHead; ++u) fs_store_unit(po, u, h, cx.hh, cx.ores);
-  }
-}
-
-__global__ __launch_bounds__(64 * kFsWaves) void k_qkv_attn_short(const uint16_t* __restrict__ xn,
-                                                                  const u32x4* __restrict__ wq,
-                                                                  const float* __restrict__ bgate,
-                                                                  const float* __restrict__ rope, int mode,
-                                                                  int nseq, int L, int T, int F,
-                                                                  uint16_t* __restrict__ O) {
-  __shared__ u32x4 smem[kFsLdsVecs];  // one LDS object: stage A, stage B, K / V^T exchange
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int j = lane & 31, hh = lane >> 5;
-  const int sl = wave & (kFsSeqs - 1), th = wave >> 2;  // sequence slot, position half
-  const int units = (nseq + kFsSeqs - 1) / kFsSeqs * kHeads;
-  const int u_begin = int(int64_t(blockIdx.x) * units / gridDim.x);
-  const int u_end = int(int64_t(blockIdx.x + 1) * units / gridDim.x);
-  FsCtx cx;
-  cx.wq = wq;
-  cx.kx_own = smem + kFsOffKx + (2 * sl + th) * 4 * 64;
-  cx.kx_other = smem + kFsOffKx + (2 * sl + (th ^ 1)) * 4 * 64;
-  cx.vx_own = smem + kFsOffVx + (2 * sl + th) * 4 * 64;
-  cx.vx_other = smem + kFsOffVx + (2 * sl + (th ^ 1)) * 4 * 64;
-  cx.L = L;
-  cx.p = 32 * th + j;
-  cx.th = th;
-  cx.hh = hh;
-  cx.lane = lane;
-  cx.wave = wave;
-  const int tok_stride = mode == 0 ? F : 1;
-  // the output row of this lane's position within its sequence (kFsDropped past the sequence end)
-  cx.qoff = cx.p < L ? cx.p * tok_stride * (kHeads * kHeadDim * 2) : kFsDropped;
-
-  fs_issue_a(u_begin % kHeads, smem, wq, wave, lane);
-  {  // rotary table [cos | sin][L][32] fp32, for this lane's position in every sequence (zero past L)
-    const bool in = cx.p < L;
-    const float* cr = rope + int64_t(in ? cx.p : 0) * 32;
-    const float* sr = cr + int64_t(L) * 32;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int i = 16 * c + 4 * g + 2 * hh;
-        cx.rope.cs[c][g] = in ? *reinterpret_cast<const float2*>(cr + i) : float2{0.f, 0.f};
-        cx.rope.sn[c][g] = in ? *reinterpret_cast<const float2*>(sr + i) : float2{0.f, 0.f};
-      }
-  }
-  FsCarry cy;
-  int h_last = 0;
-#pragma unroll 1
-  for (int u = u_begin; u < u_end;) {
-    const int grp = u / kHeads, h0 = u - grp * kHeads;
-    const int h1 = min(kHeads, h0 + (u_end - u));  // this group's heads h0 .. h1 - 1
-    if (u != u_begin) fs_flush(cx, cy, h_last);    // the previous group's last head
-    fs_issue_gate(smem + kFsOffB, wq, wave, lane);
-    const int s = grp * kFsSeqs + sl;
-    cx.active = s < nseq;  // idle waves still stage weights and meet every barrier
-    const bool valid = cx.active && cx.p < L;
-    u32x4 bx[16];  // xn of this lane's position (zero past L), natural k order
-    {
-      const u32x4* xr = reinterpret_cast<const u32x4*>(xn + (valid ? token_of(mode, s, cx.p, T, F) : 0) * kDim);
-#pragma unroll
-      for (int ks = 0; ks < 16; ++ks) bx[ks] = valid ? xr[2 * ks + hh] : zero4();
-    }
-    // O of this sequence as a buffer: token of position p at byte (token_of(p) - token_of(0)) * 1 KB
-    const int64_t tok0 = cx.active ? token_of(mode, s, 0, T, F) : 0;
-    cx.ores = buffer_rsrc(O + tok0 * (kHeads * kHeadDim),
-                          cx.active ? ((L - 1) * tok_stride + 1) * kHeads * kHeadDim * 2 : 0);
-    fs_barrier<0>();  // the gate tile, stage A of head h0 and xn
-
-    // ---- the gate tile (in stage B's buffer): rows 0..7 live in register group 0 of both half-waves
-    if (cx.active) {
-      f32x16 ga = zero16();
-#pragma unroll
-      for (int ks = 0; ks < 16; ++ks) ga = mfma32(smem[kFsOffB + ks * 64 + lane], bx[ks], ga);
-      const f32x4 bg = *reinterpret_cast<const f32x4*>(bgate + 4 * hh);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) cx.gv[r] = 1.0f / (1.0f + expf(-(ga[r] + bg[r])));
-    }
-
-    // head h0 has no previous head to finish; the others finish theirs in their stage A
-    {
-      const int next = grp * kHeads + h0 + 1;  // the next unit, if this workgroup has one
-      fs_head<false>(h0, next < u_end ? (h0 + 1) % kHeads : -1, cx, smem, bx, cy);
-    }
-#pragma unroll 1
-    for (int h = h0 + 1; h < h1; ++h) {
-      const int next = grp * kHeads + h + 1;
-      fs_head<true>(h, next < u_end ? (h + 1) % kHeads : -1, cx, smem, bx, cy);
-    }
-    h_last = h1 - 1;
-    u += h1 - h0;
-  }
-  if (u_end > u_begin) fs_flush(cx, cy, h_last);
-}
-
-// Workgroups of the fused kernel: one per CU (the kernel deals its units itself), at most one per unit.
-static int fs_grid(int nseq) {
-  const int n = device_cu_count();
-  const int units = (nseq + kFsSeqs - 1) / kFsSeqs * kHeads;
-  return units < n ? units : n;
 }
 
 void launch_qkv_attn_short(const uint16_t* xn, const uint8_t* layer, const float* rope, const SeqShape& sh,
                            uint16_t* O, hipStream_t st, const LaunchEvents& ev) {
   if (sh.nseq <= 0) return;
-  hipExtLaunchKernelGGL(k_qkv_attn_short, dim3(unsigned(fs_grid(sh.nseq))), dim3(64 * kFsWaves), 0, st, ev.start,
-                        ev.stop, 0, xn, reinterpret_cast<const u32x4*>(layer + kOffQkvg),
-                        reinterpret_cast<const float*>(layer + kOffBgate), rope, sh.mode, sh.nseq, sh.L, sh.T, sh.F,
-                        O);
+  const int C = sh.L <= 32 ? 1 : 2;
+  const int slots = device_cu_count() * (C == 1 ? 2 : 1);  // sequences the device holds
+  const auto kernel = C == 1 ? k_qkv_attn_short<1> : k_qkv_attn_short<2>;
+  hipExtLaunchKernelGGL(kernel, dim3(2u * unsigned(sh.nseq < slots ? sh.nseq : slots)), dim3(64 * kFsWaves), 0, st,
+                        ev.start, ev.stop, 0, xn, layer, rope, sh.mode, sh.nseq, sh.L, sh.T, sh.F, O);
 }
 
 }  // namespace trf

@@ -125,27 +125,36 @@ constexpr int kRopeChunks = 16;  // 16-byte chunks of a position's [cos | sin] r
 // xn of positions p0 .. p0 + 32C - 1 of sequence s, on its way to LDS as operand blocks [ct][k-step][lane]
 // (lane (j, hh): features 16k + 8hh .. +7 of row 32 ct + j); positions past L take the last one's.  A wave
 // instruction takes 4 chunks of 16 rows: 64-byte runs of global memory, 4-way conflicts in LDS.
-template <int C>
+template <int C, int NW = kTileWaves>
 struct TilePositions {
-  u32x4 x[2 * C];
+  static constexpr int N = kTileWaves / NW;  // quads of chunks a wave takes: chunks 4 (w + NW i) .. +3
+  u32x4 x[2 * C][N];
   __device__ __forceinline__ void load(const uint16_t* __restrict__ xn, int mode, int s, int p0, int L, int T, int F) {
-    const int t4 = (threadIdx.x & 63) >> 2, c4 = 4 * (threadIdx.x >> 6) + (threadIdx.x & 3);  // wave w: chunks 4w .. +3
+    const int t4 = (threadIdx.x & 63) >> 2, c4 = 4 * (threadIdx.x >> 6) + (threadIdx.x & 3);
 #pragma unroll
-    for (int i = 0; i < 2 * C; ++i)
-      x[i] = reinterpret_cast<const u32x4*>(xn + token_of(mode, s, min(p0 + 16 * i + t4, L - 1), T, F) * kDim)[c4];
+    for (int i = 0; i < 2 * C; ++i) {
+      const u32x4* const row =
+          reinterpret_cast<const u32x4*>(xn + token_of(mode, s, min(p0 + 16 * i + t4, L - 1), T, F) * kDim);
+#pragma unroll
+      for (int k = 0; k < N; ++k) x[i][k] = row[c4 + 4 * NW * k];
+    }
   }
   __device__ __forceinline__ void put(u32x4* xb) const {
     const int t4 = (threadIdx.x & 63) >> 2, c4 = 4 * (threadIdx.x >> 6) + (threadIdx.x & 3);
 #pragma unroll
     for (int i = 0; i < 2 * C; ++i)
-      xb[((i >> 1) * 16 + (c4 >> 1)) * 64 + 32 * (c4 & 1) + 16 * (i & 1) + t4] = x[i];
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const int c = c4 + 4 * NW * k;
+        xb[((i >> 1) * 16 + (c >> 1)) * 64 + 32 * (c & 1) + 16 * (i & 1) + t4] = x[i][k];
+      }
   }
 };
 
 // [cos | sin] rows (chunk c of row t at c ^ (t & 15)) of positions p0 .. p0 + 32C - 1 into LDS.
-template <int C>
+template <int C, int NW = kTileWaves>
 __device__ __forceinline__ void stage_rope(const float* __restrict__ rope, int p0, int L, u32x4* rrows) {
-  constexpr int R = 32 * C, NT = 64 * kTileWaves;
+  constexpr int R = 32 * C, NT = 64 * NW;
   const u32x4* const rp = reinterpret_cast<const u32x4*>(rope);
 #pragma unroll
   for (int i = 0; i < R * kRopeChunks / NT; ++i) {  // the table is [cos | sin][L][8 chunks]
@@ -174,28 +183,28 @@ __device__ __forceinline__ u32x4 join_halves(u32x2 lo, u32x2 hi) {
   return u32x4{x[0], y[0], x[1], y[1]};
 }
 
-// This wave's two k-steps of the gate tile (operand blocks ag; rows 0..7 live in register group 0 of both
-// half-waves) as partial sums [wave][position][head].
-template <int C>
-__device__ __forceinline__ void gate_partials(const u32x4 (&ag)[2], const u32x4* xb, float* part, int wave,
+// This wave's share of the gate tile's 16 k-steps (operand blocks ag; rows 0..7 live in register group 0 of
+// both half-waves) as partial sums [wave][position][head].
+template <int C, int NW = kTileWaves>
+__device__ __forceinline__ void gate_partials(const u32x4 (&ag)[16 / NW], const u32x4* xb, float* part, int wave,
                                               int lane) {
   const int j = lane & 31, hh = lane >> 5;
 #pragma unroll
   for (int ct = 0; ct < C; ++ct) {
     f32x16 acc = zero16();
 #pragma unroll
-    for (int i = 0; i < 2; ++i) acc = mfma32(ag[i], xb[(ct * 16 + 2 * wave + i) * 64 + lane], acc);
+    for (int i = 0; i < 16 / NW; ++i) acc = mfma32(ag[i], xb[(ct * 16 + 16 / NW * wave + i) * 64 + lane], acc);
     *reinterpret_cast<f32x4*>(part + (wave * 32 * C + 32 * ct + j) * kHeads + 4 * hh) =
         f32x4{acc[0], acc[1], acc[2], acc[3]};
   }
 }
 
 // The sigmoid gate of a head and position, once every wave's partial sums are there.
-template <int C>
+template <int C, int NW = kTileWaves>
 __device__ __forceinline__ float gate_of(const float* part, int p, int head, const float* __restrict__ bgate) {
   float g = part[p * kHeads + head];
 #pragma unroll
-  for (int w = 1; w < kTileWaves; ++w) g += part[(w * 32 * C + p) * kHeads + head];
+  for (int w = 1; w < NW; ++w) g += part[(w * 32 * C + p) * kHeads + head];
   return 1.0f / (1.0f + expf(-(g + bgate[head])));
 }
 
