@@ -160,9 +160,9 @@ struct MaskPlan {
 
 // ---------------------------------------------------------------- band split (trf_band_split.hip)
 // Per band f: RMSNorm of the frame's din_f features, Linear din_f -> kDim.  Packed weights of a band:
-// W' = W * gamma * sqrt(din) as fp32 A operands of v_mfma_f32_32x32x2_f32, [din/2 k-pairs][8 tiles][64
-// lanes] (lane l: output 32t + l%32, input 2p + l/32), then the bias [kDim].
-constexpr int kBandFrames = 32;  // frames per workgroup (4 waves, 2 output tiles each)
+// W' = W * gamma * sqrt(din) as fp32 A operands of v_mfma_f32_32x32x2_f32, four MFMAs (8 inputs) per 16 bytes
+// of a lane (the order is at k_pack_band_split), then the bias [kDim].
+constexpr int kBandFrames = 32;  // frames per workgroup (8 waves, one output tile each)
 
 struct BandPlan {
   int32_t n_bands, n_frames, width, ngroups;  // ngroups = workgroups per band
