@@ -236,13 +236,19 @@ int mask_layout(const int32_t* dins, int32_t n_bands, int32_t hidden, MaskLayout
 // Launch plan: each band is cut into jobs of at most kMaskPairs output pairs (as even as possible), and
 // the jobs are dealt to the XCDs largest first, each to the XCD with the least work so far (work of a job
 // ~ its MFMAs per frame: 16 k-steps of GEMM1 + 4 per output pair of GEMM2).  A workgroup of XCD x then
-// runs one job over kMaskFrames frames; the workgroups of one job on one XCD share its weights in L2.
+// runs one job over kMaskFrames frames (kMaskFewTile of them when there are few); the workgroups of one job on one XCD share its weights in L2.
 unsigned mask_plan(const MaskLayout& L, int32_t n_frames, trf::MaskPlan& p) {
   p = trf::MaskPlan{};
   p.hidden = L.hidden;
   p.n_frames = n_frames;
   p.F = L.n_bands;
-  p.ntb = (n_frames + trf::kMaskFrames - 1) / trf::kMaskFrames;
+  int jobs_few = 0;
+  for (int d : L.din) jobs_few += (mask_npairs(d) + trf::kMaskFewPairs - 1) / trf::kMaskFewPairs;
+  const bool few = n_frames <= trf::kMaskFewFrames && jobs_few <= trf::kMaskMaxJobs;
+  const int most_pairs = few ? trf::kMaskFewPairs : trf::kMaskPairs;  // per job
+  p.few = few;
+  const int tile = few ? trf::kMaskFewTile : trf::kMaskFrames;
+  p.ntb = (n_frames + tile - 1) / tile;
   p.b1_off = uint32_t(L.b1_off);
   struct Job {
     uint32_t code;
@@ -256,7 +262,7 @@ unsigned mask_plan(const MaskLayout& L, int32_t n_frames, trf::MaskPlan& p) {
     p.col[f] = uint32_t(col);
     p.din[f] = uint32_t(L.din[f]);
     col += L.din[f];
-    const int np = mask_npairs(L.din[f]), nj = mask_njobs(L.din[f]);
+    const int np = mask_npairs(L.din[f]), nj = (np + most_pairs - 1) / most_pairs;
     for (int q = 0, p0 = 0; q < nj; ++q) {
       const int n = np / nj + (q < np % nj ? 1 : 0);
       jobs.push_back(Job{uint32_t(f) | uint32_t(n) << 8 | uint32_t(p0) << 16, 16 + 4 * n});

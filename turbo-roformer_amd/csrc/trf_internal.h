@@ -134,6 +134,9 @@ constexpr int kMaxBands = 64;
 constexpr int kMaskMaxJobs = 192;
 constexpr int kMaskPairs = 6;      // output pairs per job: the largest that fits the LDS stages
 constexpr int kMaskFrames = 128;   // frames per workgroup (4 waves x 32)
+constexpr int kMaskFewTile = 32;      // frames per workgroup of a launch of at most kMaskFewFrames
+constexpr int kMaskFewFrames = 256;  // the two kernels meet at ~340 frames (fp16) and ~330 (split)
+constexpr int kMaskFewPairs = 3;      // output pairs per job of such a launch
 constexpr int kMaskW1Blocks = 32;  // blocks of W1 per hidden tile
 constexpr int kXcds = 8;           // workgroups are dealt round-robin over the 8 XCDs
 
@@ -141,9 +144,10 @@ enum MaskPrecision { kMaskSplit = 0, kMaskFp16 = 1 };
 
 // Everything a mask-head launch needs besides the pointers, passed by value.  A job is (band, first
 // output pair p0, np pairs); the workgroups of XCD x run jobs job[xcd_start[x] .. xcd_start[x+1]) one
-// after the other, each over ntb blocks of kMaskFrames frames.
+// after the other, each over ntb blocks of kMaskFrames frames (few: kMaskFewTile).
 struct MaskPlan {
   int32_t hidden, n_frames, F, width, ntb;
+  int32_t few;                      // the kernel for few frames (k_mask_few)
   uint32_t b1_off;                  // byte offset of b1 in the packed buffer
   uint32_t xcd_start[kXcds + 1];
   uint32_t job[kMaskMaxJobs];       // band | np << 8 | p0 << 16

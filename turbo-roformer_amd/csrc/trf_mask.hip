@@ -278,6 +278,167 @@ __global__ __launch_bounds__(64 * kMaskWaves) __attribute__((amdgpu_waves_per_eu
   static_assert(kMaskPairs == 6, "one case per pair count");
 }
 
+// ============================================================ few frames
+// The kernel above gives a workgroup 128 frames of a job and runs its 32 hidden tiles one after the other:
+// with few frames its launch is one round of that chain on a fraction of the CUs (47 us at 101 frames, fp16, 68
+// workgroups).  Here a workgroup is 32 frames of a job and its 8 waves share out the hidden tiles (wave w:
+// tiles w, w + 8, ...): a wave runs both GEMMs of a tile on its own, weights from L2 into registers, tanh's
+// registers as GEMM2's operands, and the waves' GEMM2 sums are added through LDS at the end.  No barrier in
+// between.  Same products and splits as above; the weights pass through L2 once per 32 frames instead of
+// 128, which is why it is for few frames.  62 bands, us a call, 128-frame workgroups and these: 49.7 and 27.6 at
+// 101 frames, 51.9 and 40.6 at 200, 54.8 and 58.0 at 384 (fp16); 84.5 and 42.2, 91.1 and 68.6, 97.9 and 107.3
+// (split).  Loading 4 operands ahead instead of 14 cost 18% at 101 frames: with one workgroup on a CU the
+// weights' latency from the memory-side cache is what bounds it.
+constexpr int kMaskFewWaves = 8;
+
+template <bool SPLIT, int NP>
+__device__ __forceinline__ void mask_few_job(const MaskPlan& p, const float* __restrict__ X,
+                                             const uint8_t* __restrict__ packed, float* __restrict__ mask, int band,
+                                             int p0, int n0, u32x4* smem) {
+  constexpr int PARTS = SPLIT ? 2 : 1, U = 16 + 4 * NP;  // operands of a hidden tile
+  constexpr int D = SPLIT ? U / 4 : U / 2;               // loaded ahead (14 KB a wave at 3 pairs)
+  u32x4* const xb = smem;  // [part][16 k-steps][64 lanes]
+  u32x4* const red = smem + PARTS * 16 * 64;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int j = lane & 31, hh = lane >> 5;
+  const int din = p.din[band], npairs = (din + 31) >> 5, nht = p.hidden >> 5;
+  const int tblocks = kMaskW1Blocks + 8 * npairs;  // 1 KB blocks of a hidden tile
+  const auto wres = buffer_rsrc(packed + size_t(p.wofs_kb[band]) * 1024, nht * tblocks * 1024);
+  // Operand u of hidden tile t: GEMM1 k-step u, then GEMM2 (pair, a / g, k-step) in order.
+  auto load = [&](int t, int u, int part) __attribute__((always_inline)) {
+    return __builtin_bit_cast(
+        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                   wres, lane * 16, (t * tblocks + (u < 16 ? 2 * u : kMaskW1Blocks + 8 * p0 + 2 * (u - 16)) + part) * 1024, 0));
+  };
+  u32x4 w[D][PARTS];
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) w[i][q] = load(min(wave, nht - 1), i, q);
+  // wave w normalises frames 4w .. 4w + 3: lane l holds inputs 4l .. 4l + 3 of a row
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = 4 * wave + i;
+    const f32x4 x = *reinterpret_cast<const f32x4*>(
+        X + (int64_t(min(n0 + t, p.n_frames - 1)) * p.F + band) * kDim + 4 * lane);
+    float ss = fmaf(x[0], x[0], fmaf(x[1], x[1], fmaf(x[2], x[2], x[3] * x[3])));
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
+    const float inv = 1.0f / fmaxf(sqrtf(ss), 1e-12f);
+    u32x2 hi, lo;
+    uint32_t h, l;
+    split_f16(x[0] * inv * kMaskNormScale, x[1] * inv * kMaskNormScale, h, l);
+    hi[0] = h, lo[0] = l;
+    split_f16(x[2] * inv * kMaskNormScale, x[3] * inv * kMaskNormScale, h, l);
+    hi[1] = h, lo[1] = l;
+    const int at = 2 * ((lane >> 2) * 64 + 32 * (lane >> 1 & 1) + t) + (lane & 1);
+    reinterpret_cast<u32x2*>(xb)[at] = hi;
+    if (SPLIT) reinterpret_cast<u32x2*>(xb + 16 * 64)[at] = lo;
+  }
+  __syncthreads();
+  const float* const b1 = reinterpret_cast<const float*>(packed + p.b1_off) + size_t(band) * p.hidden;
+  f32x16 acc[2 * NP];
+#pragma unroll
+  for (int i = 0; i < 2 * NP; ++i) acc[i] = zero16();
+#pragma unroll 1
+  for (int t = wave; t < nht; t += kMaskFewWaves) {
+    const int tn = min(t + kMaskFewWaves, nht - 1);  // the next tile (past the last: any, unused)
+    auto advance = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q) w[u % D][q] = u + D < U ? load(t, u + D, q) : load(tn, u + D - U, q);
+    };
+    f32x16 h0, h1 = zero16();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(b1 + 32 * t + row_of_group(g, hh));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) h0[4 * g + r] = b[r];
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const u32x4 xh = xb[k * 64 + lane];
+      f32x16& c0 = k & 1 ? h1 : h0;
+      f32x16& c1 = k & 1 ? h0 : h1;
+      c0 = mfma32h(w[k % D][0], xh, c0);
+      if constexpr (SPLIT) {
+        c1 = mfma32h(w[k % D][0], xb[(16 + k) * 64 + lane], c1);
+        c0 = mfma32h(w[k % D][1], xh, c0);
+      }
+      advance(k);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    u32x4 hh_[2], hl_[2];  // tanh as GEMM2 operands (hidden k-steps 0 and 1 of the tile), hi and lo
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      uint32_t h, l;
+      split_f16(tanh_f32(h0[2 * v] + h1[2 * v]), tanh_f32(h0[2 * v + 1] + h1[2 * v + 1]), h, l);
+      hh_[v >> 2][v & 3] = h;
+      hl_[v >> 2][v & 3] = l;
+    }
+#pragma unroll
+    for (int u = 16; u < U; ++u) {
+      const int k = u & 1;
+      f32x16& c = acc[(u - 16) >> 1];
+      c = mfma32h(w[u % D][0], hh_[k], c);
+      if constexpr (SPLIT) {
+        c = mfma32h(w[u % D][0], hl_[k], c);
+        c = mfma32h(w[u % D][1], hh_[k], c);
+      }
+      advance(u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // The waves' sums, one output pair at a time: [wave][a / g][register group][lane].
+  const float* const b2 = reinterpret_cast<const float*>(packed + p.b2_off[band]);
+  const int pad = 32 * npairs;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if (i) __syncthreads();
+#pragma unroll
+    for (int ag = 0; ag < 2; ++ag)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& c = acc[2 * i + ag];
+        red[((wave * 2 + ag) * 4 + g) * 64 + lane] =
+            __builtin_bit_cast(u32x4, f32x4{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]});
+      }
+    __syncthreads();
+    if (wave < 4) {  // register group `wave`
+      const int c = 32 * (p0 + i) + row_of_group(wave, hh);
+      f32x4 a = *reinterpret_cast<const f32x4*>(b2 + c), g = *reinterpret_cast<const f32x4*>(b2 + pad + c);
+#pragma unroll
+      for (int v = 0; v < kMaskFewWaves; ++v) {
+        a += __builtin_bit_cast(f32x4, red[(v * 8 + wave) * 64 + lane]);
+        g += __builtin_bit_cast(f32x4, red[(v * 8 + 4 + wave) * 64 + lane]);
+      }
+      f32x4 m;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] = a[r] / (1.0f + __expf(-g[r]));
+      if (n0 + j < p.n_frames && c < din)
+        *reinterpret_cast<f32x4*>(mask + int64_t(n0 + j) * p.width + p.col[band] + c) = m;
+    }
+  }
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(64 * kMaskFewWaves, 2) void k_mask_few(const float* __restrict__ X,
+                                                                    const uint8_t* __restrict__ packed,
+                                                                    float* __restrict__ mask, const MaskPlan p) {
+  __shared__ u32x4 smem[(SPLIT ? 2 : 1) * 16 * 64 + kMaskFewWaves * 8 * 64];
+  const int xcd = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
+  const int slot = k / p.ntb, n0 = (k - slot * p.ntb) * kMaskFewTile;
+  const int first = p.xcd_start[xcd];
+  if (slot >= int(p.xcd_start[xcd + 1]) - first) return;
+  const uint32_t job = p.job[first + slot];
+  const int band = job & 0xff, np = (job >> 8) & 0xff, p0 = job >> 16;
+  switch (np) {
+    case 1: mask_few_job<SPLIT, 1>(p, X, packed, mask, band, p0, n0, smem); break;
+    case 2: mask_few_job<SPLIT, 2>(p, X, packed, mask, band, p0, n0, smem); break;
+    default: mask_few_job<SPLIT, 3>(p, X, packed, mask, band, p0, n0, smem); break;
+  }
+  static_assert(kMaskFewPairs == 3, "one case per pair count");
+}
+
 // ============================================================ packing
 // Items of a band: (tile j, block, lane) -> one 16-byte lane slot of the layout in trf_internal.h.
 //   W1 block 2s + hl, lane l: rows 32j + l%32, inputs 16s + 8(l/32) + e, times gamma (natural k order).
@@ -345,6 +506,11 @@ void launch_pack_mask_band(const float* w1, const float* gamma, const float* b1,
 
 void launch_mask_head(const float* X, const uint8_t* packed, float* mask, const MaskPlan& plan, unsigned grid,
                       int precision, hipStream_t st) {
+  if (plan.few) {
+    hipLaunchKernelGGL(precision == kMaskFp16 ? k_mask_few<false> : k_mask_few<true>, dim3(grid),
+                       dim3(64 * kMaskFewWaves), 0, st, X, packed, mask, plan);
+    return;
+  }
   if (precision == kMaskFp16)
     hipLaunchKernelGGL(k_mask_head<false>, dim3(grid), dim3(64 * kMaskWaves), 0, st, X, packed, mask, plan);
   else
