@@ -12,6 +12,7 @@ bitwise the same sums as the host loop).
 
 from __future__ import annotations
 
+import math
 from collections.abc import Callable
 
 import numpy as np
@@ -42,8 +43,9 @@ def hamming(n: int) -> np.ndarray:
     """Symmetric Hamming window 0.54 - 0.46 cos(2 pi k / (n-1)), float32; ones(1) for n = 1."""
     if n == 1:
         return np.ones(1, np.float32)
-    k = np.arange(n, dtype=np.float64)
-    return (0.54 - 0.46 * np.cos(2.0 * np.pi * k / (n - 1))).astype(np.float32)
+    # the float64 steps of the formula in order, on torch's threads (a 17 s chunk: 1.1 ms, numpy's cosine 8)
+    k = torch.arange(n, dtype=torch.float64, device="cpu")
+    return k.mul_(2.0 * math.pi).div_(n - 1).cos_().mul_(-0.46).add_(0.54).float().numpy()
 
 
 def overlap_add(
@@ -103,7 +105,7 @@ def overlap_add_device(
     C = min(chunk, n)
     starts = chunk_starts(n, C, step_for(C, overlap))
     dev = x.device
-    w = torch.from_numpy(hamming(C)).to(dev)
+    w = None
     acc = torch.zeros(2, n, dtype=torch.float32, device=dev)
     wsum = torch.zeros(n, dtype=torch.float32, device=dev)
     per = len(starts) if batch <= 0 else batch
@@ -111,6 +113,8 @@ def overlap_add_device(
         group = starts[b0 : b0 + per]
         y = run(torch.stack([x[:, s : s + C] for s in group]).contiguous()).float().contiguous()
         L = min(C, y.shape[-1])
+        if w is None:  # formed on the host while the device runs the first chunks
+            w = torch.from_numpy(hamming(C)).pin_memory().to(dev, non_blocking=True)
         _hip.overlap_add(y, L, group, w, acc, wsum)
         if progress is not None:
             for k in range(len(group)):
