@@ -66,22 +66,22 @@ struct MaskOps {
   }
 };
 
-// One stage.  LAST: tanh and GEMM2 of the last hidden tile only.  Otherwise: pre := tile u-1 (+ b1),
-// tanh(pre) into the GEMM2 B operands, one value after each GEMM1 unit, then GEMM2(u-1); b1 of tile u is
-// loaded for the next stage, and dma(q) issues this wave's q-th direct-to-LDS block of the next stage
+// One stage.  pre holds tile u-1's pre-activations.  LAST: tanh and GEMM2 of the last hidden tile only.
+// Otherwise: tanh(pre) into the GEMM2 B operands, one value after each GEMM1 unit, then GEMM2(u-1) with
+// the sums of tile u's pre-activations (the two chains and b1) between its MFMAs: at the start of the next
+// stage they would stand alone, 64 instructions of the wave's single SIMD.  dma(q) issues this wave's q-th direct-to-LDS block of the next stage
 // after unit q.  (Issued all at once, the next stage's 40-80 KB per workgroup outrun what a CU keeps in
 // flight and the wave stalls in issue before its MFMAs; spread over the first units, they stream under
 // them and land before the stage ends.)  Each unit's operand blocks are read one unit ahead.
 template <bool SPLIT, int NP, bool LAST, typename Dma>
 __device__ __forceinline__ void mask_stage(const u32x4* L, int u, const float* b1, const u32x4 (&xh)[16],
-                                           const u32x4 (&xl)[16], f32x16& hA, f32x16& hB, f32x4 (&b1v)[4],
-                                           f32x16 (&acc)[2 * NP], int lane, int hh, Dma&& dma) {
+                                           const u32x4 (&xl)[16], float (&pre)[16], f32x16 (&acc)[2 * NP],
+                                           int lane, int hh, Dma&& dma) {
   using O = MaskOps<SPLIT, NP>;
   constexpr int K0 = LAST ? O::U1 : 0;  // first unit of the stage
   static_assert(O::NB / kMaskWaves <= O::U, "one DMA block per unit");
-  float pre[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) pre[r] = hA[r] + hB[r] + b1v[r >> 2][r & 3];
+  f32x16 hA = zero16(), hB = zero16();
+  f32x4 b1v[4];
   if (!LAST) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) b1v[g] = *reinterpret_cast<const f32x4*>(b1 + 32 * u + 8 * g + 4 * hh);
@@ -133,6 +133,12 @@ __device__ __forceinline__ void mask_stage(const u32x4* L, int u, const float* b
         g = mfma32h(cur[2], hbl[t], g);
         a = mfma32h(cur[1], hbh[t], a);
         g = mfma32h(cur[3], hbh[t], g);
+      }
+      if (!LAST) {
+        constexpr int N = 2 * NP;  // units of GEMM2
+#pragma unroll
+        for (int r = 16 * (k - O::U1) / N; r < 16 * (k - O::U1 + 1) / N; ++r)
+          pre[r] = hA[r] + hB[r] + b1v[r >> 2][r & 3];
       }
     }
     if (!LAST && k < O::NB / kMaskWaves) dma(k);
@@ -223,23 +229,22 @@ __device__ __forceinline__ void mask_job(const MaskPlan& p, const float* __restr
       xl[s][q] = l;
     }
 
-  f32x16 hA = zero16(), hB = zero16();
-  f32x4 b1v[4];
+  float pre[16];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) b1v[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < 16; ++r) pre[r] = 0.f;
   // Stages go in pairs so that each one's LDS buffer is a compile-time constant (the compiler then tells
   // operand reads from the direct-to-LDS loads into the other buffer and does not wait for those).
 #pragma clang loop unroll(disable)
   for (int u = 0; u < nht; u += 2) {
     stage_barrier();
-    mask_stage<SPLIT, NP, false>(lds0, u, b1, xh, xl, hA, hB, b1v, acc, lane, hh,
+    mask_stage<SPLIT, NP, false>(lds0, u, b1, xh, xl, pre, acc, lane, hh,
                                  [&](int q) { issue(u + 1, lds1, q); });
     stage_barrier();
-    mask_stage<SPLIT, NP, false>(lds1, u + 1, b1, xh, xl, hA, hB, b1v, acc, lane, hh,
+    mask_stage<SPLIT, NP, false>(lds1, u + 1, b1, xh, xl, pre, acc, lane, hh,
                                  [&](int q) { issue(u + 2, lds0, q); });
   }
   stage_barrier();
-  mask_stage<SPLIT, NP, true>(lds0, nht, b1, xh, xl, hA, hB, b1v, acc, lane, hh, [](int) {});
+  mask_stage<SPLIT, NP, true>(lds0, nht, b1, xh, xl, pre, acc, lane, hh, [](int) {});
 
   if (!valid) return;
   float* mrow = mask + int64_t(n) * p.width + p.col[band];
