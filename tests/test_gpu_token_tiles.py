@@ -97,3 +97,25 @@ def test_fused_block_matches_its_halves(hip, precision, T, F):
         stack.ff_block(want, 1, T, F, layer)
     torch.cuda.synchronize()
     assert snr_db((want - X).cpu().numpy(), (got - X).cpu().numpy()) >= 60.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,spiked", [(128, False), (129, False), (383, True), (385, False), (640, True), (641, False)])
+def test_attention_query_blocks(hip, T, spiked):
+    """Time attention at the edges of its 128- and 256-query workgroups; spiked: one key scores 100 above the
+    rest for half a query tile, so the workgroup redoes its sweep with the guarded shift.  Floor as in
+    test_gpu_ops.py."""
+    F, g = 2, torch.Generator().manual_seed(T)
+    sd = weights.init_state_dict(CFG, seed=3, init="normal")
+    w = ok.bf16_weights(folded.fold(sd, 1)[0])
+    xn = ok.l2_rows(torch.randn(T * F, 256, generator=g)).to(torch.bfloat16)
+    Q, K, Vt, G = ok.qkv_rope(xn, w["W"], w["b_gate"], w["freqs"], 0, 1, T, F)
+    if spiked:
+        K[:, :, :, 350, :] = 4.0
+        Q[:, :, :, 96:112, :] = 100.0 / (64 * 16.0) * 4.0
+    want = ok.attention(Q, K, Vt, G, 0, 1, T, F)
+    O = torch.empty(T * F, 512, dtype=torch.bfloat16, device=DEV)
+    print(f"attention query blocks T={T} spiked={spiked}", flush=True)
+    _hip.attention(Q.to(DEV), K.to(DEV), Vt.to(DEV), G.to(DEV), O, 0, 1, T, F)
+    torch.cuda.synchronize()
+    assert_bf16_close(want, O, "O", min_snr=48)

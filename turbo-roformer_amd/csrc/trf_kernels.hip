@@ -397,14 +397,13 @@ __device__ __forceinline__ void attn_store(const f32x16 (&o)[2], int q, int L, i
 // shift it is rounded like the others, and dividing by the sum of the weights P.V actually applied makes
 // up for that: against exact attention the result is within ~0.5 dB of the reference's arithmetic on
 // peaked rows, where the sum of e leaves it 2-3 dB below.
-// One workgroup = one (sequence, head) and 4 waves x 64 queries; each wave holds two 32-query column
-// tiles, so every K or V^T operand read from LDS feeds two MFMAs.  Tiles of 64 keys of K and V^T stream
+// One workgroup = one (sequence, head) and 4 waves x 32 QT queries; with QT = 2 a wave holds two 32-query
+// column tiles, so every K or V^T operand read from LDS feeds two MFMAs (QT = 1: see launch_attention).  Tiles of 64 keys of K and V^T stream
 // through a ring of LDS buffers, loaded global->LDS directly (V^T with the XOR swizzle of its 16-byte
 // chunks applied through each lane's source address, for bank-conflict-free operand reads).  Only the
 // last key tile can hold keys >= L, so the masked code runs once.
 constexpr int kAttWaves = 4;
-constexpr int kAttQT = 2;                       // 32-query column tiles per wave
-constexpr int kAttBlockQ = kAttWaves * 32 * kAttQT;  // queries per workgroup
+constexpr int att_block_q(int QT) { return kAttWaves * 32 * QT; }  // queries per workgroup of QT column tiles a wave
 
 // Physical 16-byte chunk of logical chunk c in LDS row R is c ^ chunk_swz(R).  Operand reads touch
 // rows R0..R0+31 at one logical chunk; with 64 four-byte banks (two 128-byte rows per bank sweep) this
@@ -503,18 +502,18 @@ __device__ __forceinline__ void attn_half(const u32x4 (&ka)[4], const u32x4 (&qb
 }
 
 // One 64-key tile: per 32-key half, scores and probabilities for both query tiles, then P.V.
-template <bool FIRST, bool MASK, bool SAFE>
+template <bool FIRST, bool MASK, bool SAFE, int QT>
 __device__ __forceinline__ void attn_tile(const u32x4* __restrict__ Kl, const u32x4* __restrict__ Vl,
-                                          const u32x4 (&qb)[kAttQT][4], int key0, int L, int j, int hh,
-                                          const u32x4& ones, f32x16 (&negc)[kAttQT], f32x4 (&psum)[kAttQT],
-                                          f32x16 (&o)[kAttQT][2]) {
+                                          const u32x4 (&qb)[QT][4], int key0, int L, int j, int hh,
+                                          const u32x4& ones, f32x16 (&negc)[QT], f32x4 (&psum)[QT],
+                                          f32x16 (&o)[QT][2]) {
 #pragma unroll
   for (int kh = 0; kh < 2; ++kh) {
     u32x4 ka[4];
     load_k_half(Kl, kh, j, hh, ka);
-    u32x4 p0[kAttQT], p1[kAttQT];
+    u32x4 p0[QT], p1[QT];
 #pragma unroll
-    for (int qt = 0; qt < kAttQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       if (FIRST && kh == 0)
         attn_half<true, false, SAFE>(ka, qb[qt], 0, L, hh, ones, negc[qt], psum[qt], o[qt], p0[qt], p1[qt]);
       else
@@ -527,7 +526,7 @@ __device__ __forceinline__ void attn_tile(const u32x4* __restrict__ Kl, const u3
       const u32x4 v0 = Vl[d * 8 + ((4 * kh + hh) ^ chunk_swz(d))];
       const u32x4 v1 = Vl[d * 8 + ((4 * kh + 2 + hh) ^ chunk_swz(d))];
 #pragma unroll
-      for (int qt = 0; qt < kAttQT; ++qt) {
+      for (int qt = 0; qt < QT; ++qt) {
         o[qt][dt] = mfma32(v0, p0[qt], o[qt][dt]);
         o[qt][dt] = mfma32(v1, p1[qt], o[qt][dt]);
       }
@@ -540,7 +539,8 @@ __device__ __forceinline__ void attn_tile(const u32x4* __restrict__ Kl, const u3
 // 2 for a K tile, 4 for K + V), and the barrier makes every wave's share visible.
 constexpr int kAttBufs = 3;
 
-__global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+template <int QT>
+__global__ __launch_bounds__(256, 4 - QT) void k_attn_long(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                                                    const uint16_t* __restrict__ Vt, const float* __restrict__ G,
                                                    uint16_t* __restrict__ O, int mode, int L, int Lpad, int T,
                                                    int F, int nqb) {
@@ -557,12 +557,12 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
   // K and V^T of this (sequence, head) as buffer resources for the direct-to-LDS tile loads.
   const __amdgpu_buffer_rsrc_t Kh = buffer_rsrc(K + int64_t(sh) * Lpad * kHeadDim, Lpad * kHeadDim * 2);
   const __amdgpu_buffer_rsrc_t Vh = buffer_rsrc(Vt + int64_t(sh) * kHeadDim * Lpad, Lpad * kHeadDim * 2);
-  const int q0 = qblk * kAttBlockQ + wave * 32 * kAttQT;
+  const int q0 = qblk * att_block_q(QT) + wave * 32 * QT;
   const bool active = q0 < L;  // idle waves still stage tiles and meet every barrier
 
-  u32x4 qb[kAttQT][4];
+  u32x4 qb[QT][4];
 #pragma unroll
-  for (int qt = 0; qt < kAttQT; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     const int q = q0 + 32 * qt + j;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
@@ -571,12 +571,12 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
 
   const int nkt = Lpad / 64;  // >= 2: this kernel runs for L > 64
   const u32x4 ones = rowsum_ones(lane);
-  f32x4 psum[kAttQT];
-  f32x16 negc[kAttQT], o[kAttQT][2];
+  f32x4 psum[QT];
+  f32x16 negc[QT], o[QT][2];
   auto sweep = [&](auto safe_tag) {
     constexpr bool SAFE = decltype(safe_tag)::value;
 #pragma unroll
-    for (int qt = 0; qt < kAttQT; ++qt) {
+    for (int qt = 0; qt < QT; ++qt) {
       psum[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
       negc[qt] = o[qt][0] = o[qt][1] = zero16();
     }
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
       stage_k_tile(Kh, kAttBufs - 1, Lpad, lds[kAttBufs - 1][0], wave, lane);
       stage_v_tile(Vh, kAttBufs - 1, Lpad, lds[kAttBufs - 1][1], wave, lane);
     }
-    if (active) attn_tile<true, false, SAFE>(lds[0][0], lds[0][1], qb, 0, L, j, hh, ones, negc, psum, o);
+    if (active) attn_tile<true, false, SAFE, QT>(lds[0][0], lds[0][1], qb, 0, L, j, hh, ones, negc, psum, o);
     for (int kt = 1; kt < nkt - 1; ++kt) {
       if (kt + kAttBufs - 2 < nkt)  // K and V: 4 loads per younger tile in flight
         vmcnt_barrier<4 * (kAttBufs - 2)>();
@@ -603,12 +603,12 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
         stage_v_tile(Vh, kt + kAttBufs - 1, Lpad, lds[b][1], wave, lane);
       }
       if (active)
-        attn_tile<false, false, SAFE>(lds[kt % kAttBufs][0], lds[kt % kAttBufs][1], qb, 0, L, j, hh, ones, negc,
+        attn_tile<false, false, SAFE, QT>(lds[kt % kAttBufs][0], lds[kt % kAttBufs][1], qb, 0, L, j, hh, ones, negc,
                                       psum, o);
     }
     vmcnt_barrier<0>();
     if (active)
-      attn_tile<false, true, SAFE>(lds[(nkt - 1) % kAttBufs][0], lds[(nkt - 1) % kAttBufs][1], qb, (nkt - 1) * 64, L,
+      attn_tile<false, true, SAFE, QT>(lds[(nkt - 1) % kAttBufs][0], lds[(nkt - 1) % kAttBufs][1], qb, (nkt - 1) * 64, L,
                                    j, hh, ones, negc, psum, o);
   };
   sweep(std::integral_constant<bool, false>{});
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
   // by the whole workgroup (it streams K/V through the shared LDS ring), if any of its rows failed.
   bool bad = false;
 #pragma unroll
-  for (int qt = 0; qt < kAttQT; ++qt) {
+  for (int qt = 0; qt < QT; ++qt) {
     bad |= !(psum_of_query(psum[qt], j) <= kAttSafeSum);
     float om = 0.f;
 #pragma unroll
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_long(const uint16_t* __restrict
   if (__syncthreads_or(active && bad)) sweep(std::integral_constant<bool, true>{});
   if (!active) return;
 #pragma unroll
-  for (int qt = 0; qt < kAttQT; ++qt)
+  for (int qt = 0; qt < QT; ++qt)
     attn_store(o[qt], q0 + 32 * qt + j, L, s, h, hh, mode, T, F, G, psum_of_query(psum[qt], j), O);
 }
 
@@ -704,8 +704,15 @@ void launch_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* Vt, 
                           sh.mode, nsh, sh.L,
                        sh.T, sh.F);
   } else {
-    const int nqb = (sh.L + kAttBlockQ - 1) / kAttBlockQ;
-    hipExtLaunchKernelGGL(k_attn_long, dim3(sh.nseq * kHeads * nqb), dim3(64 * kAttWaves), 0, st, ev.start, ev.stop,
+    // Two column tiles a wave share each operand read of a 256-query workgroup; one makes a 128-query
+    // workgroup, for an odd number of 128-query blocks, whose last 256-query one would run half empty. us at
+    // 62 bands, QT = 2 and 1: L = 101 11.2 and 9.6, 257 30.8 and 24.2, 384 35.3 and 30.3, 520 58.3 and 55.9,
+    // 640 65.3 and 64.5, 896 114 and 114 (even numbers of blocks: 200 18.6 and 19.2, 800 102 and 101).
+    const int blocks = (sh.L + att_block_q(1) - 1) / att_block_q(1);
+    const int QT = blocks % 2 && blocks <= 5 ? 1 : 2;
+    const int nqb = (sh.L + att_block_q(QT) - 1) / att_block_q(QT);
+    const auto kernel = QT == 1 ? k_attn_long<1> : k_attn_long<2>;
+    hipExtLaunchKernelGGL(kernel, dim3(sh.nseq * kHeads * nqb), dim3(64 * kAttWaves), 0, st, ev.start, ev.stop,
                           0, Q, K, Vt, G, O,
                        sh.mode, sh.L, sh.Lpad, sh.T, sh.F, nqb);
   }
