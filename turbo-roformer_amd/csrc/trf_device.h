@@ -80,10 +80,10 @@ __device__ __forceinline__ float halfwave_max(float x) {
 // stay in scalar registers.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
-// ============================================================ LDS weight streaming
-// Weights are packed as 1 KB operand blocks (one MFMA A operand: 64 lanes x 16 B).  A workgroup
-// streams the blocks of one stage into LDS with direct global->LDS loads, double-buffered: while the
-// waves compute on stage s from one buffer, the blocks of stage s+1 land in the other.
+// ============================================================ direct-to-LDS streaming
+// Weights are packed as 1 KB operand blocks (one MFMA A operand: 64 lanes x 16 B). The mask head streams the
+// blocks of one stage into LDS with direct global->LDS loads, double-buffered; the attention kernel its K and
+// V^T tiles, and the token-tile kernels their rows.
 //
 // The direct loads are buffer loads with an LDS destination (buffer_load_dwordx4 ... lds).  The compiler
 // counts global_load_lds among the LDS operations, so after one it can only wait lgkmcnt(0) before an
@@ -100,11 +100,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
 __device__ __forceinline__ void buffer_load_lds16(__amdgpu_buffer_rsrc_t r, int voff, u32x4* lds_base) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_base, 16, voff, 0, 0,
                                            0);
-}
-
-// One operand block (src_block wave-uniform) into LDS.
-__device__ __forceinline__ void lds_load_block(const u32x4* __restrict__ src_block, u32x4* lds_block, int lane) {
-  buffer_load_lds16(buffer_rsrc(src_block, kTileBytes), lane * 16, lds_block);
 }
 
 // All of this thread's outstanding global loads (direct-to-LDS ones included) have landed, and every
