@@ -135,8 +135,8 @@ constexpr int kMaskMaxJobs = 192;
 constexpr int kMaskPairs = 6;      // output pairs per job: the largest that fits the LDS stages
 constexpr int kMaskFrames = 128;   // frames per workgroup (4 waves x 32)
 constexpr int kMaskFewTile = 32;      // frames per workgroup of a launch of at most kMaskFewFrames
-constexpr int kMaskFewFrames = 256;  // the two kernels meet at ~340 frames (fp16) and ~330 (split)
-constexpr int kMaskFewPairs = 3;      // output pairs per job of such a launch
+constexpr int kMaskFewFrames = 256;  // 62 bands: the two kernels meet at ~350 frames (fp16) and ~310 (split)
+constexpr int kMaskFewPairs = 4;      // output pairs per job of such a launch (a wave per a or g tile)
 constexpr int kMaskW1Blocks = 32;  // blocks of W1 per hidden tile
 constexpr int kXcds = 8;           // workgroups are dealt round-robin over the 8 XCDs
 

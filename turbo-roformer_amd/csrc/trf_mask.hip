@@ -20,7 +20,9 @@
 //               accumulator order (W2 is packed with its k order permuted to match).
 // Stage 0 multiplies its W2 blocks (tile 0) by tanh(0) = 0 exactly; a last stage runs tanh and GEMM2 of
 // the last tile.  b1 is added with the tanh; the GEMM2 accumulators start at b2; the GLU is the epilogue.
-#include "trf_device.h"
+#include "trf_tiles.h"
+
+#include <type_traits>
 
 namespace trf {
 
@@ -284,164 +286,218 @@ __global__ __launch_bounds__(64 * kMaskWaves) __attribute__((amdgpu_waves_per_eu
 }
 
 // ============================================================ few frames
-// The kernel above gives a workgroup 128 frames of a job and runs its 32 hidden tiles one after the other:
-// with few frames its launch is one round of that chain on a fraction of the CUs (47 us at 101 frames, fp16, 68
-// workgroups).  Here a workgroup is 32 frames of a job and its 8 waves share out the hidden tiles (wave w:
-// tiles w, w + 8, ...): a wave runs both GEMMs of a tile on its own, weights from L2 into registers, tanh's
-// registers as GEMM2's operands, and the waves' GEMM2 sums are added through LDS at the end.  No barrier in
-// between.  Same products and splits as above; the weights pass through L2 once per 32 frames instead of
-// 128, which is why it is for few frames.  62 bands, us a call, 128-frame workgroups and these: 49.7 and 27.6 at
-// 101 frames, 51.9 and 40.6 at 200, 54.8 and 58.0 at 384 (fp16); 84.5 and 42.2, 91.1 and 68.6, 97.9 and 107.3
-// (split).  Loading 4 operands ahead instead of 14 cost 18% at 101 frames: with one workgroup on a CU the
-// weights' latency from the memory-side cache is what bounds it.
+// The kernel above gives a workgroup 128 frames of a job and runs its hidden tiles one after the other: with
+// few frames its launch is one round of that chain on a fraction of the CUs.  Here a workgroup is 32 frames of
+// a job and its 8 waves take the hidden tiles in groups of 8: wave w forms tile 8g + w and leaves its tanh in
+// LDS as GEMM2 operands, and then owns one GEMM2 accumulator (wave 2i: the a tile of output pair i, wave
+// 2i + 1: its g tile), over the 8 tiles of the group before.  So one barrier per group, weights from L2 into
+// registers, and every sum in the order of the kernel above: a frame's mask is the same, bit for bit, whichever
+// kernel runs and however many frames are in the launch.
+// 62 bands, us a call, 128-frame workgroups and these: 44 and 22 at 64 frames, 45 and 27 at 128 (fp16); 80 and
+// 31, 82 and 45 (split).  fp16 runs two workgroups a CU (128 registers a wave; one, with weights loaded 8
+// k-steps ahead: 21 and 30), split one.  Waves that each ran both GEMMs of their tiles and added their sums at
+// the end, without barriers, took 24 at 128 frames (fp16) and 40 (split), with masks that differed in the last
+// bits from those of the same frames in a larger launch.
 constexpr int kMaskFewWaves = 8;
+constexpr int kMaskFewHb = 2 * 2 * kMaskFewWaves * 64;  // hidden operands of two groups, one part
+static_assert(2 * kMaskFewPairs <= kMaskFewWaves, "a wave per GEMM2 accumulator");
 
-template <bool SPLIT, int NP>
-__device__ __forceinline__ void mask_few_job(const MaskPlan& p, const float* __restrict__ X,
-                                             const uint8_t* __restrict__ packed, float* __restrict__ mask, int band,
-                                             int p0, int n0, u32x4* smem) {
-  constexpr int PARTS = SPLIT ? 2 : 1, U = 16 + 4 * NP;  // operands of a hidden tile
-  constexpr int D = SPLIT ? U / 4 : U / 2;               // loaded ahead (14 KB a wave at 3 pairs)
-  u32x4* const xb = smem;  // [part][16 k-steps][64 lanes]
-  u32x4* const red = smem + PARTS * 16 * 64;
+template <bool SPLIT>
+__global__ __launch_bounds__(64 * kMaskFewWaves, SPLIT ? 2 : 4) void k_mask_few(const float* __restrict__ X,
+                                                                    const uint8_t* __restrict__ packed,
+                                                                    float* __restrict__ mask, const MaskPlan p) {
+  constexpr int PARTS = SPLIT ? 2 : 1;
+  constexpr int D = 4;  // k-steps the weights of both GEMMs are loaded ahead (fp16, 8: one workgroup a CU)
+  __shared__ u32x4 smem[PARTS * (16 * 64 + kMaskFewHb) + 8];
+  u32x4* const xb = smem;                    // [part][16 k-steps][64 lanes]; at the end the g tiles
+  u32x4* const hb = smem + PARTS * 16 * 64;  // [group & 1][tile][k-step][part][64 lanes]; first the fp32 rows
+  float* const inv = reinterpret_cast<float*>(smem + PARTS * (16 * 64 + kMaskFewHb));
+  static_assert(kMaskFewHb >= kMaskFewTile * 64, "the rows fit");
+  const int xcd = blockIdx.x % kXcds, kb = blockIdx.x / kXcds;
+  const int slot = kb / p.ntb, n0 = (kb - slot * p.ntb) * kMaskFewTile;
+  const int first = p.xcd_start[xcd];
+  if (slot >= int(p.xcd_start[xcd + 1]) - first) return;
+  const uint32_t job = p.job[first + slot];
+  const int band = job & 0xff, np = (job >> 8) & 0xff, p0 = job >> 16;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int j = lane & 31, hh = lane >> 5;
   const int din = p.din[band], npairs = (din + 31) >> 5, nht = p.hidden >> 5;
   const int tblocks = kMaskW1Blocks + 8 * npairs;  // 1 KB blocks of a hidden tile
+  const int groups = (nht + kMaskFewWaves - 1) / kMaskFewWaves;
+  const bool gemm2 = wave < 2 * np;  // this wave owns an accumulator (the others repeat the last pair's loads)
+  const int w2_block = kMaskW1Blocks + 8 * (p0 + min(wave >> 1, np - 1)) + 4 * (wave & 1);
   const auto wres = buffer_rsrc(packed + size_t(p.wofs_kb[band]) * 1024, nht * tblocks * 1024);
-  // Operand u of hidden tile t: GEMM1 k-step u, then GEMM2 (pair, a / g, k-step) in order.
-  auto load = [&](int t, int u, int part) __attribute__((always_inline)) {
-    return __builtin_bit_cast(
-        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                   wres, lane * 16, (t * tblocks + (u < 16 ? 2 * u : kMaskW1Blocks + 8 * p0 + 2 * (u - 16)) + part) * 1024, 0));
+  auto load = [&](int t, int block) __attribute__((always_inline)) {  // (a tile past the last: the last, unused)
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                         wres, lane * 16, (min(t, nht - 1) * tblocks + block) * 1024, 0));
   };
-  u32x4 w[D][PARTS];
+  // k-step s of GEMM1 on the wave's tile of group g; k-step s of GEMM2 on group g (tile s / 2, its half s % 2)
+  u32x4 w1[D][PARTS], w2[D][PARTS];
+  auto load1 = [&](int g, int s, int q) __attribute__((always_inline)) {
+    return load(kMaskFewWaves * g + wave, 2 * s + q);
+  };
+  auto load2 = [&](int g, int s, int q) __attribute__((always_inline)) {
+    return load(kMaskFewWaves * g + (s >> 1), w2_block + 2 * (s & 1) + q);
+  };
 #pragma unroll
-  for (int i = 0; i < D; ++i)
+  for (int s = 0; s < D; ++s)
 #pragma unroll
-    for (int q = 0; q < PARTS; ++q) w[i][q] = load(min(wave, nht - 1), i, q);
-  // wave w normalises frames 4w .. 4w + 3: lane l holds inputs 4l .. 4l + 3 of a row
+    for (int q = 0; q < PARTS; ++q) w1[s][q] = load1(0, s, q);
+  // wave w loads frames 4w .. 4w + 3 (past the last one: the last): lane l inputs 4l .. 4l + 3
+  f32x4 x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    x[i] = *reinterpret_cast<const f32x4*>(
+        X + (int64_t(min(n0 + 4 * wave + i, p.n_frames - 1)) * p.F + band) * kDim + 4 * lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) hb[row_chunk(4 * wave + i, lane)] = __builtin_bit_cast(u32x4, x[i]);
+#pragma unroll
+  for (int s = 0; s < D; ++s)
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) w2[s][q] = load2(0, s, q);
+  f32x16 acc;
+  {
+    const float* const b2 = reinterpret_cast<const float*>(packed + p.b2_off[band]) + (wave & 1) * 32 * npairs +
+                            32 * (p0 + min(wave >> 1, np - 1));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(b2 + row_of_group(g, hh));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[4 * g + r] = b[r];
+    }
+  }
+  lds_barrier();
+  if (wave == 0) {  // lane (j, hh) sums the squares of its half of frame j's inputs in mask_job's order
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+      const f32x4 v = __builtin_bit_cast(f32x4, hb[row_chunk(j, 4 * (c >> 1) + 2 * hh + (c & 1))]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
+    }
+    ss += __shfl_xor(ss, 32);
+    if (hh == 0) inv[j] = 1.0f / fmaxf(sqrtf(ss), 1e-12f);
+  }
+  lds_barrier();
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int t = 4 * wave + i;
-    const f32x4 x = *reinterpret_cast<const f32x4*>(
-        X + (int64_t(min(n0 + t, p.n_frames - 1)) * p.F + band) * kDim + 4 * lane);
-    float ss = fmaf(x[0], x[0], fmaf(x[1], x[1], fmaf(x[2], x[2], x[3] * x[3])));
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
-    const float inv = 1.0f / fmaxf(sqrtf(ss), 1e-12f);
+    const float sc = inv[t];
     u32x2 hi, lo;
     uint32_t h, l;
-    split_f16(x[0] * inv * kMaskNormScale, x[1] * inv * kMaskNormScale, h, l);
+    split_f16(x[i][0] * sc * kMaskNormScale, x[i][1] * sc * kMaskNormScale, h, l);
     hi[0] = h, lo[0] = l;
-    split_f16(x[2] * inv * kMaskNormScale, x[3] * inv * kMaskNormScale, h, l);
+    split_f16(x[i][2] * sc * kMaskNormScale, x[i][3] * sc * kMaskNormScale, h, l);
     hi[1] = h, lo[1] = l;
     const int at = 2 * ((lane >> 2) * 64 + 32 * (lane >> 1 & 1) + t) + (lane & 1);
     reinterpret_cast<u32x2*>(xb)[at] = hi;
     if (SPLIT) reinterpret_cast<u32x2*>(xb + 16 * 64)[at] = lo;
   }
-  __syncthreads();
+  lds_barrier();
   const float* const b1 = reinterpret_cast<const float*>(packed + p.b1_off) + size_t(band) * p.hidden;
-  f32x16 acc[2 * NP];
+  f32x16 h0, h1;
+  // GEMM1 of group g (ONE) beside GEMM2 of group g - 1 (TWO).
+  auto steps = [&](auto one_tag, auto two_tag, int g) __attribute__((always_inline)) {
+    constexpr bool ONE = decltype(one_tag)::value, TWO = decltype(two_tag)::value;
+    const u32x4* const hg = hb + ((g - 1) & 1) * (PARTS * kMaskFewHb / 2);
+    u32x4 xo[2][PARTS], ho[2][PARTS];
+    auto read = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 2 * NP; ++i) acc[i] = zero16();
-#pragma unroll 1
-  for (int t = wave; t < nht; t += kMaskFewWaves) {
-    const int tn = min(t + kMaskFewWaves, nht - 1);  // the next tile (past the last: any, unused)
-    auto advance = [&](int u) __attribute__((always_inline)) {
-#pragma unroll
-      for (int q = 0; q < PARTS; ++q) w[u % D][q] = u + D < U ? load(t, u + D, q) : load(tn, u + D - U, q);
+      for (int q = 0; q < PARTS; ++q) {
+        if (ONE) xo[s & 1][q] = xb[(q * 16 + s) * 64 + lane];
+        if (TWO) ho[s & 1][q] = hg[(s * PARTS + q) * 64 + lane];
+      }
     };
-    f32x16 h0, h1 = zero16();
+    read(0);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4 b = *reinterpret_cast<const f32x4*>(b1 + 32 * t + row_of_group(g, hh));
-#pragma unroll
-      for (int r = 0; r < 4; ++r) h0[4 * g + r] = b[r];
-    }
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const u32x4 xh = xb[k * 64 + lane];
-      f32x16& c0 = k & 1 ? h1 : h0;
-      f32x16& c1 = k & 1 ? h0 : h1;
-      c0 = mfma32h(w[k % D][0], xh, c0);
-      if constexpr (SPLIT) {
-        c1 = mfma32h(w[k % D][0], xb[(16 + k) * 64 + lane], c1);
-        c0 = mfma32h(w[k % D][1], xh, c0);
+    for (int s = 0; s < 16; ++s) {
+      if (s + 1 < 16) read(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      u32x4 (&xs)[PARTS] = xo[s & 1];
+      u32x4 (&hs)[PARTS] = ho[s & 1];
+      if constexpr (ONE) {
+        f32x16& c0 = s & 1 ? h1 : h0;  // mask_stage's chains
+        f32x16& c1 = s & 1 ? h0 : h1;
+        c0 = mfma32h(w1[s % D][0], xs[0], s == 0 || (!SPLIT && s == 1) ? zero16() : c0);
+        if constexpr (SPLIT) {
+          c1 = mfma32h(w1[s % D][0], xs[1], s == 0 ? zero16() : c1);
+          c0 = mfma32h(w1[s % D][1], xs[0], c0);
+        }
       }
-      advance(k);
+      if constexpr (TWO) {
+        acc = mfma32h(w2[s % D][0], hs[0], acc);
+        if constexpr (SPLIT) {
+          acc = mfma32h(w2[s % D][0], hs[1], acc);
+          acc = mfma32h(w2[s % D][1], hs[0], acc);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < PARTS; ++q) {
+        if (ONE) w1[s % D][q] = s + D < 16 ? load1(g, s + D, q) : load1(g + 1, s + D - 16, q);
+        if (TWO) w2[s % D][q] = s + D < 16 ? load2(g - 1, s + D, q) : load2(g, s + D - 16, q);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    u32x4 hh_[2], hl_[2];  // tanh as GEMM2 operands (hidden k-steps 0 and 1 of the tile), hi and lo
+  };
+  constexpr std::integral_constant<bool, true> yes{};
+  constexpr std::integral_constant<bool, false> no{};
+#pragma unroll 1
+  for (int g = 0; g < groups; ++g) {
+    const int t = kMaskFewWaves * g + wave;
+    f32x4 b1v[4];
+    auto load_b1 = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      uint32_t h, l;
-      split_f16(tanh_f32(h0[2 * v] + h1[2 * v]), tanh_f32(h0[2 * v + 1] + h1[2 * v + 1]), h, l);
-      hh_[v >> 2][v & 3] = h;
-      hl_[v >> 2][v & 3] = l;
-    }
+      for (int r = 0; r < 4; ++r)
+        b1v[r] = *reinterpret_cast<const f32x4*>(b1 + 32 * min(t, nht - 1) + row_of_group(r, hh));
+    };
+    if (SPLIT) load_b1();
+    if (gemm2 && g)
+      steps(yes, yes, g);
+    else
+      steps(yes, no, g);
+    if (!SPLIT) load_b1();  // (16 registers it does not have during the products)
+    u32x4* const hw = hb + (g & 1) * (PARTS * kMaskFewHb / 2) + wave * 2 * PARTS * 64 + lane;
 #pragma unroll
-    for (int u = 16; u < U; ++u) {
-      const int k = u & 1;
-      f32x16& c = acc[(u - 16) >> 1];
-      c = mfma32h(w[u % D][0], hh_[k], c);
-      if constexpr (SPLIT) {
-        c = mfma32h(w[u % D][0], hl_[k], c);
-        c = mfma32h(w[u % D][1], hh_[k], c);
+    for (int ks = 0; ks < 2; ++ks) {  // tanh as operands of the tile's two k-steps, zero past the last tile
+      u32x4 hi = zero4(), lo = zero4();
+      if (t < nht) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = 8 * ks + 2 * v;
+          uint32_t h, l;
+          split_f16(tanh_f32(h0[r] + h1[r] + b1v[r >> 2][r & 3]),
+                    tanh_f32(h0[r + 1] + h1[r + 1] + b1v[r >> 2][(r & 3) + 1]), h, l);
+          hi[v] = h;
+          lo[v] = l;
+        }
       }
-      advance(u);
-      __builtin_amdgcn_sched_barrier(0);
+      hw[ks * PARTS * 64] = hi;
+      if (SPLIT) hw[(ks * PARTS + 1) * 64] = lo;
     }
+    lds_barrier();  // the group's operands are there, the ones before have been read
   }
-  // The waves' sums, one output pair at a time: [wave][a / g][register group][lane].
-  const float* const b2 = reinterpret_cast<const float*>(packed + p.b2_off[band]);
-  const int pad = 32 * npairs;
+  if (gemm2) steps(no, yes, groups);
+  // The GLU: the g tile of a pair passes from its wave to the a tile's through LDS (xb has been read).
+  u32x4* const red = xb + (wave >> 1) * 4 * 64 + lane;
+  static_assert(kMaskFewPairs * 4 <= 16, "the g tiles fit");
+  if (gemm2 && (wave & 1)) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    if (i) __syncthreads();
-#pragma unroll
-    for (int ag = 0; ag < 2; ++ag)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[2 * i + ag];
-        red[((wave * 2 + ag) * 4 + g) * 64 + lane] =
-            __builtin_bit_cast(u32x4, f32x4{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]});
-      }
-    __syncthreads();
-    if (wave < 4) {  // register group `wave`
-      const int c = 32 * (p0 + i) + row_of_group(wave, hh);
-      f32x4 a = *reinterpret_cast<const f32x4*>(b2 + c), g = *reinterpret_cast<const f32x4*>(b2 + pad + c);
-#pragma unroll
-      for (int v = 0; v < kMaskFewWaves; ++v) {
-        a += __builtin_bit_cast(f32x4, red[(v * 8 + wave) * 64 + lane]);
-        g += __builtin_bit_cast(f32x4, red[(v * 8 + 4 + wave) * 64 + lane]);
-      }
-      f32x4 m;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) m[r] = a[r] / (1.0f + __expf(-g[r]));
-      if (n0 + j < p.n_frames && c < din)
-        *reinterpret_cast<f32x4*>(mask + int64_t(n0 + j) * p.width + p.col[band] + c) = m;
-    }
+    for (int g = 0; g < 4; ++g)
+      red[g * 64] = __builtin_bit_cast(u32x4, f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]});
   }
-}
-
-template <bool SPLIT>
-__global__ __launch_bounds__(64 * kMaskFewWaves, 2) void k_mask_few(const float* __restrict__ X,
-                                                                    const uint8_t* __restrict__ packed,
-                                                                    float* __restrict__ mask, const MaskPlan p) {
-  __shared__ u32x4 smem[(SPLIT ? 2 : 1) * 16 * 64 + kMaskFewWaves * 8 * 64];
-  const int xcd = blockIdx.x % kXcds, k = blockIdx.x / kXcds;
-  const int slot = k / p.ntb, n0 = (k - slot * p.ntb) * kMaskFewTile;
-  const int first = p.xcd_start[xcd];
-  if (slot >= int(p.xcd_start[xcd + 1]) - first) return;
-  const uint32_t job = p.job[first + slot];
-  const int band = job & 0xff, np = (job >> 8) & 0xff, p0 = job >> 16;
-  switch (np) {
-    case 1: mask_few_job<SPLIT, 1>(p, X, packed, mask, band, p0, n0, smem); break;
-    case 2: mask_few_job<SPLIT, 2>(p, X, packed, mask, band, p0, n0, smem); break;
-    default: mask_few_job<SPLIT, 3>(p, X, packed, mask, band, p0, n0, smem); break;
+  lds_barrier();
+  if (!gemm2 || (wave & 1) || n0 + j >= p.n_frames) return;
+  float* const mrow = mask + int64_t(n0 + j) * p.width + p.col[band];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int c = 32 * (p0 + (wave >> 1)) + row_of_group(g, hh);  // mask columns c..c+3 of the band
+    if (c >= din) continue;
+    const f32x4 gv = __builtin_bit_cast(f32x4, red[g * 64]);
+    f32x4 m;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) m[r] = acc[4 * g + r] / (1.0f + __expf(-gv[r]));
+    *reinterpret_cast<f32x4*>(mrow + c) = m;
   }
-  static_assert(kMaskFewPairs == 3, "one case per pair count");
 }
 
 // ============================================================ packing
