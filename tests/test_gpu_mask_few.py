@@ -49,7 +49,7 @@ def test_mask_head_few_frames(hip, precision, floor, hidden, n_frames):
 @pytest.mark.parametrize("hidden", [64, 320, 1024])  # 2 hidden tiles (6 waves have none), 10 (two groups), 32
 def test_mask_rows_do_not_depend_on_the_launch(hip, precision, hidden):
     """A frame's mask is the same bits in a launch of few frames and in one of 3,200, which the other kernel
-    takes.  Widths of 1, 2, 3 and
+    takes (4 bands: 1.7 times the load per CU up to which the kernel for few frames runs).  Widths of 1, 2, 3 and
     9 output pairs: the last is jobs of 3 pairs in one kernel, of 5 and 4 in the other."""
     dims, n = (8, 40, 96, 260), 3200
     g = torch.Generator().manual_seed(hidden)

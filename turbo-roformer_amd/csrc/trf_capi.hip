@@ -233,18 +233,28 @@ int mask_layout(const int32_t* dins, int32_t n_bands, int32_t hidden, MaskLayout
   return TRF_OK;
 }
 
-// Launch plan: each band is cut into jobs of at most kMaskPairs output pairs (as even as possible), and
-// the jobs are dealt to the XCDs largest first, each to the XCD with the least work so far (work of a job
-// ~ its MFMAs per frame: 16 k-steps of GEMM1 + 4 per output pair of GEMM2).  A workgroup of XCD x then
-// runs one job over kMaskFrames frames (kMaskFewTile of them when there are few); the workgroups of one job on one XCD share its weights in L2.
+// Launch plan: each band is cut into jobs of at most kMaskPairs (few frames: kMaskFewPairs) output pairs, as
+// even as possible, and the jobs are dealt to the XCDs largest first, each to the XCD with the least work so
+// far (work of a job ~ its MFMAs per frame: 16 k-steps of GEMM1 + 4 per output pair of GEMM2).  A workgroup of
+// XCD x then runs one job over kMaskFrames (kMaskFewTile) frames; the workgroups of one job on one XCD share
+// its weights in L2.
+// The kernel for few frames takes a launch while its work per CU is at most kMaskFewLoad times the longest job
+// of the other kernel, whose launch is at least that long however few workgroups it has.
 unsigned mask_plan(const MaskLayout& L, int32_t n_frames, trf::MaskPlan& p) {
   p = trf::MaskPlan{};
   p.hidden = L.hidden;
   p.n_frames = n_frames;
   p.F = L.n_bands;
-  int jobs_few = 0;
-  for (int d : L.din) jobs_few += (mask_npairs(d) + trf::kMaskFewPairs - 1) / trf::kMaskFewPairs;
-  const bool few = n_frames <= trf::kMaskFewFrames && jobs_few <= trf::kMaskMaxJobs;
+  int64_t jobs_few = 0, work_few = 0, longest = 0;
+  for (int d : L.din) {
+    const int np = mask_npairs(d), nj = mask_njobs(d), nf = (np + trf::kMaskFewPairs - 1) / trf::kMaskFewPairs;
+    jobs_few += nf;
+    work_few += 16 * nf + 4 * np;
+    longest = std::max<int64_t>(longest, 16 + 4 * ((np + nj - 1) / nj));
+  }
+  work_few *= (n_frames + trf::kMaskFewTile - 1) / trf::kMaskFewTile;
+  const bool few =
+      jobs_few <= trf::kMaskMaxJobs && double(work_few) <= trf::kMaskFewLoad * double(longest * trf::device_cu_count());
   const int most_pairs = few ? trf::kMaskFewPairs : trf::kMaskPairs;  // per job
   p.few = few;
   const int tile = few ? trf::kMaskFewTile : trf::kMaskFrames;

@@ -134,9 +134,15 @@ constexpr int kMaxBands = 64;
 constexpr int kMaskMaxJobs = 192;
 constexpr int kMaskPairs = 6;      // output pairs per job: the largest that fits the LDS stages
 constexpr int kMaskFrames = 128;   // frames per workgroup (4 waves x 32)
-constexpr int kMaskFewTile = 32;      // frames per workgroup of a launch of at most kMaskFewFrames
-constexpr int kMaskFewFrames = 256;  // 62 bands: the two kernels meet at ~350 frames (fp16) and ~310 (split)
-constexpr int kMaskFewPairs = 4;      // output pairs per job of such a launch (a wave per a or g tile)
+// The kernel for few frames (k_mask_few): frames per workgroup, output pairs per job (a wave per a or g tile),
+// and up to what load per CU it is taken (the rule is at mask_plan).  Both kernels' us on either side of the line,
+// few and 128-frame, fp16 then split: 62 bands 256 frames (load 1.45) 38 and 45, 71 and 80, 320 (1.8) 43 and 46,
+// 90 and 86; 20 bands of 512: 192 (1.5) 32 and 46, 62 and 82, 224 (1.75) 44 and 46, 87 and 81; 64 bands of 96:
+// 192 (1.5) 30 and 35, 55 and 63, 288 (2.25) 40 and 36, 81 and 68; 29 bands (hidden 512) 640 (1.4) 22 and 27,
+// 40 and 44, 1024 (2.3) 29 and 27, 57 and 45.
+constexpr int kMaskFewTile = 32;
+constexpr int kMaskFewPairs = 4;
+constexpr double kMaskFewLoad = 1.6;
 constexpr int kMaskW1Blocks = 32;  // blocks of W1 per hidden tile
 constexpr int kXcds = 8;           // workgroups are dealt round-robin over the 8 XCDs
 
@@ -147,7 +153,7 @@ enum MaskPrecision { kMaskSplit = 0, kMaskFp16 = 1 };
 // after the other, each over ntb blocks of kMaskFrames frames (few: kMaskFewTile).
 struct MaskPlan {
   int32_t hidden, n_frames, F, width, ntb;
-  int32_t few;                      // the kernel for few frames (k_mask_few)
+  int32_t few;                      // the kernel for few frames
   uint32_t b1_off;                  // byte offset of b1 in the packed buffer
   uint32_t xcd_start[kXcds + 1];
   uint32_t job[kMaskMaxJobs];       // band | np << 8 | p0 << 16
