@@ -56,6 +56,28 @@ def test_gemm_gelu_widths(hip, n, n_out):
 
 
 @pytest.mark.gpu
+def test_gemm_gelu_is_as_close_as_erff(hip):
+    """Zero weights, so the outputs are the GELU of the biases: 2^20 normal ones, of which 0.5 x (1 + erff(x /
+    sqrt 2)) in float32 rounds 2.4e-5 to the wrong bf16 (+- 5e-6: sampling).  A&S 7.1.26 rounds 9.6e-5."""
+    n_out = 1 << 18
+    xn = torch.zeros(1, 256, dtype=torch.bfloat16, device=DEV)
+    Wp = _hip.pack_weight(torch.zeros(n_out, 256, dtype=torch.bfloat16, device=DEV))
+    wrong = 0
+    for seed in range(4):
+        b = torch.randn(n_out, generator=torch.Generator().manual_seed(seed))
+        b[:8] = torch.tensor([0.0, -0.0, float("inf"), -float("inf"), 1e30, -1e30, 75.0, -75.0])
+        H = torch.empty(1, n_out, dtype=torch.bfloat16, device=DEV)
+        print(f"gemm_gelu of biases, seed {seed}", flush=True)
+        _hip.gemm_gelu(xn, Wp, b.to(DEV), H)
+        x = b.double()
+        exact = 0.5 * x * (1 + torch.erf(x / 2**0.5))
+        exact[3] = 0.0  # the limit (0.5 inf 0)
+        wrong += int((H[0].cpu() != exact.float().to(torch.bfloat16)).sum())
+        assert torch.equal(H[0, :8].cpu().float(), exact[:8].to(torch.bfloat16).float())
+    assert wrong <= 40, f"{wrong} of 2^20 outputs round to the wrong bf16"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["ff_fp16", "ff_split", "bf16"])
 @pytest.mark.parametrize("n", [1, 33, 8192, 8193])
 def test_feed_forward_tiles(hip, precision, n):
