@@ -78,6 +78,25 @@ def test_gemm_gelu_is_as_close_as_erff(hip):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_out,n", [(32, 16385), (64, 32773)])
+def test_gemm_gelu_narrow(hip, n_out, n):
+    """One or two weight tiles and more than 16,384 tokens a tile: the kernel without LDS, the same bits as the
+    other one's on a part of the tokens (the last workgroup and the last wave are partial)."""
+    W, b = _weight(n_out, 256, 7)
+    xn = (rand_x(n, 71) * 0.5).to(torch.bfloat16)
+    Wp = _hip.pack_weight(W.to(DEV))
+    H = torch.full((n + 1, n_out), 7.0, dtype=torch.bfloat16, device=DEV)
+    print(f"gemm_gelu narrow n_out={n_out} n={n}", flush=True)
+    _hip.gemm_gelu(xn.to(DEV), Wp, b.to(DEV), H[:n])
+    assert bool((H[n] == 7.0).all())
+    part = slice(n - 4001, n)
+    Hp = torch.empty(4001, n_out, dtype=torch.bfloat16, device=DEV)
+    _hip.gemm_gelu(xn[part].contiguous().to(DEV), Wp, b.to(DEV), Hp)
+    assert torch.equal(H[part], Hp)
+    assert_bf16_close(ok.gemm_gelu(xn[part], W, b), Hp, "H", min_snr=50)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["ff_fp16", "ff_split", "bf16"])
 @pytest.mark.parametrize("n", [1, 33, 8192, 8193])
 def test_feed_forward_tiles(hip, precision, n):

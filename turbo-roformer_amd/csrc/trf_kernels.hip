@@ -1060,8 +1060,51 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_gelu(const uint16_t
   }
 }
 
+// The same for a narrow output of many tokens: a wave is 32 tokens, from global memory to global memory, without
+// LDS or barriers.  Above, one or two of the eight waves have a weight tile and the others only move rows; that
+// costs when the rows no longer come and go under one round of workgroups.  us, above and here: n_out = 32 8.2 and
+// 8.3 at 18,786 tokens, 14.4 and 8.1 at 52,700, 29.0 and 13.8 at 105,462; n_out = 64 9.3 and 10 at 32,674, 14.9 and
+// 10.8 at 52,700, 29.6 and 19.9 at 105,462.  Same sums, so the same bits.
+__global__ __launch_bounds__(256) void k_gemm_gelu_narrow(const uint16_t* __restrict__ xn, const u32x4* __restrict__ wq,
+                                                          const float* __restrict__ b1, int n_out,
+                                                          uint16_t* __restrict__ H, int64_t n) {
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int j = lane & 31, hh = lane >> 5;
+  const int64_t tok = (int64_t(blockIdx.x) * 4 + wave) * 32 + j;
+  const bool valid = tok < n;
+  const u32x4* const xr = reinterpret_cast<const u32x4*>(xn + (valid ? tok : n - 1) * kDim);
+  u32x4 x[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) x[k] = xr[2 * k + hh];
+  uint16_t* const hr = H + tok * n_out;
+#pragma unroll 1
+  for (int t = 0; t < n_out / 32; ++t) {
+    const u32x4* const w = wq + t * 16 * 64 + lane;
+    f32x16 acc;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(b1 + 32 * t + row_of_group(g, hh));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[4 * g + r] = b[r];
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc = mfma32(w[k * 64], x[k], acc);
+    if (!valid) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<u32x2*>(hr + 32 * t + row_of_group(g, hh)) =
+          u32x2{pk_bf16(gelu_op(acc[4 * g]), gelu_op(acc[4 * g + 1])),
+                pk_bf16(gelu_op(acc[4 * g + 2]), gelu_op(acc[4 * g + 3]))};
+  }
+}
+
 void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* bias, int n_out, uint16_t* H,
                       int64_t n, hipStream_t st) {
+  if (n_out <= 64 && n > 512 * int64_t(n_out)) {
+    hipLaunchKernelGGL(k_gemm_gelu_narrow, dim3(unsigned((n + 127) / 128)), dim3(256), 0, st, xn,
+                       reinterpret_cast<const u32x4*>(w_packed), bias, n_out, H, n);
+    return;
+  }
   const int C = token_tiles(n);
   const auto kernel = C == 1 ? k_gemm_gelu<1> : k_gemm_gelu<2>;
   hipLaunchKernelGGL(kernel, dim3(unsigned((n + 32 * C - 1) / (32 * C))), dim3(64 * kTileWaves), 0, st, xn,
