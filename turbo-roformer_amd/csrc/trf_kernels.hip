@@ -862,8 +862,8 @@ __device__ __forceinline__ void add_rows(const u32x4* rowbuf, f32x16 (&acc)[C], 
 // X[tok] += A[tok] . W^T (+ b); xn[tok] = X / max(|X|, eps), for any A width K (a multiple of 16) and a
 // weight W [256][K] packed in natural k order (launch_pack, kPack32Natural); xn may be null (not written).
 // A is staged in panels of 512 columns (a row's chunks past K are dropped).  HBM-bound (378 MB at
-// 105,462 tokens and K = 512: 74 us at the rate of a copy; 486 MB and 95 us at K = 1024): 85 and 160 us, of
-// 269 and 512 for waves that read A and W from global memory as they multiplied, with no LDS.
+// 105,462 tokens and K = 512: 74 us at the rate of a copy; 486 MB and 95 us at K = 1024): 76 and 127 us, of
+// 221 and 422 for waves that read A and W from global memory as they multiplied, with no LDS.
 // (kernels.cpp:542-586)
 template <int C>
 __global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_res_norm(const uint16_t* __restrict__ A, int K,
@@ -962,7 +962,12 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_res_norm(const uint
 
 void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
                           uint16_t* xn, int64_t n, float eps, hipStream_t st, const LaunchEvents& ev) {
-  const int C = token_tiles(n);
+  // One panel of A: a tile's two memory phases leave little for the weights to bound, and 32-token tiles, whose
+  // accumulators and X rows need no scratch, overlap them better.  us, 64- and 32-token tiles, K = 512: 22.1 and
+  // 18.4 at 18,786 tokens, 23.2 and 24.5 at 24,800 (the one size where they lose: the 64-token tiles are one
+  // round), 51.5 and 42.1 at 52,700, 91 and 76 at 105,462; K = 128: 60 and 52 there.  More panels: K = 768 57 and 54
+  // at 52,700 but 27 and 29.6 at 24,800; K = 1024 63 and 68, 127 and 137 at 105,462.
+  const int C = K <= 512 ? 1 : token_tiles(n);
   const auto kernel = C == 1 ? k_gemm_res_norm<1> : k_gemm_res_norm<2>;
   hipExtLaunchKernelGGL(kernel, dim3(unsigned((n + 32 * C - 1) / (32 * C))), dim3(64 * kTileWaves), 0, st, ev.start,
                         ev.stop, 0, A, K, reinterpret_cast<const u32x4*>(w_packed), bias, X, xn, n, eps);
