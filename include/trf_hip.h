@@ -46,7 +46,9 @@
 extern "C" {
 #endif
 
-#define TRF_ABI_VERSION 8
+/* Packed weights (trf_pack_layer, trf_pack_weight, trf_pack_mask_head, trf_pack_band_split) are in the kernels'
+ * own order, which belongs to this version: pack again after trf_abi_version() changes. */
+#define TRF_ABI_VERSION 9
 
 #define TRF_DIM 256
 #define TRF_HEADS 8

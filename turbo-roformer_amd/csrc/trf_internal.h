@@ -41,8 +41,9 @@ constexpr size_t kOffFf2Lo = kOffFf1Lo + kSzFf1;
 // fp16 W1 and W2 (32x32 register order, fp16(hi + lo)) for the fp16 feed-forward.
 constexpr size_t kOffFf1F16 = kOffFf2Lo + kSzFf2;
 constexpr size_t kOffFf2F16 = kOffFf1F16 + kSzFf1;
-// The packed size callers allocate is the ABI's; what the tiles above do not take (a second W_out, and W1 and
-// W2 once more) is unused.
+// The packed size is one that callers allocate and tests pin; what the tiles above do not take (a second W_out,
+// and W1 and W2 once more) is unused.  A change of order or offsets here, or of the other packed weights, raises
+// TRF_ABI_VERSION.
 constexpr size_t kLayerBytes = kOffFf2F16 + kSzFf2 + kSzOut + kSzFf1 + kSzFf2;
 
 // Feed-forward arithmetic (the trf_precision values of trf_hip.h).
