@@ -531,7 +531,7 @@ int trf_ff_block(float* X, int32_t batch, int32_t T, int32_t F, const void* pack
     return fail(TRF_ERR_WORKSPACE, "workspace is %zu bytes, need %zu", workspace_bytes, w.bytes);
   hipStream_t st = as_hip(stream);
   const int64_t n = int64_t(batch) * T * F;
-  trf::launch_ff(static_cast<const uint8_t*>(packed_layer), X, nullptr, n, precision, 1e-12f, st);
+  trf::launch_ff(static_cast<const uint8_t*>(packed_layer), X, n, precision, 1e-12f, st);
   return check_launch("feed_forward");
 }
 

@@ -107,7 +107,7 @@ void launch_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* Vt, 
 void launch_qkv_attn_short(const uint16_t* xn, const uint8_t* layer, const float* rope, const SeqShape& sh,
                            uint16_t* O, hipStream_t st, const LaunchEvents& ev = {});
 // Per-op GEMMs on a standalone weight packed by launch_pack in natural k order (kPack32Natural):
-// X += A [n][K] . W^T (+ bias), xn = X / max(|X|, eps) (W [256][K]); H = gelu_erf(xn . W^T + bias)
+// X += A [n][K] . W^T (+ bias), xn = X / max(|X|, eps) unless xn is null (W [256][K]); H = gelu(xn . W^T + bias)
 // (W [n_out][256], n_out a multiple of 32).
 void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
                           uint16_t* xn, int64_t n, float eps, hipStream_t st, const LaunchEvents& ev = {});
@@ -117,10 +117,8 @@ void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* 
 // FfPrecision value for the two FF GEMMs.
 void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision,
                       float eps, hipStream_t st, const LaunchEvents& ev = {});
-// Fused FF1 + GELU + FF2 + residual + norm on X (updated in place, its norm computed in the kernel);
-// xn is written as X / |X|.
-// In these three xn may be null: it is then not written.
-void launch_ff(const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision, float eps, hipStream_t st);
+// Fused norm + FF1 + GELU + FF2 + residual on X (updated in place).
+void launch_ff(const uint8_t* layer, float* X, int64_t n, int ff_precision, float eps, hipStream_t st);
 
 // ---------------------------------------------------------------- mask head (trf_mask.hip)
 // Final norm + one MLP per band (Linear dim -> hidden, tanh, Linear hidden -> 2 din, GLU).

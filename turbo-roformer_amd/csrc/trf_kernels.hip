@@ -820,9 +820,9 @@ __device__ __forceinline__ float inv_norm(const float* ssq, int t, float eps) {
   return 1.0f / fmaxf(sqrtf(((p[0] + p[1]) + (p[2] + p[3])) + ((q[0] + q[1]) + (q[2] + q[3]))), eps);
 }
 
-// The end of a tile: acc (tile `wave` of every token's features) -> X rows and, normalised, xn rows.
-// `rowbuf` holds the tile's fp32 rows; every wave has met since its last use, and since put_ssq.
-template <int C>
+// The end of a tile: acc (tile `wave` of every token's features) -> X rows and, normalised, xn rows (NORM).
+// `rowbuf` holds the tile's fp32 rows; every wave has met since its last use, and since put_ssq (NORM).
+template <int C, bool NORM>
 __device__ __forceinline__ void store_tile(const f32x16 (&acc)[C], u32x4* rowbuf, const float* ssq, float eps,
                                            __amdgpu_buffer_rsrc_t xres, __amdgpu_buffer_rsrc_t nres, int wave,
                                            int lane) {
@@ -841,8 +841,9 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[C], u32x4* rowbuf
     const int t = wave * RW + i;
     const u32x4 v = rowbuf[row_chunk(t, lane)];
     const f32x4 x = __builtin_bit_cast(f32x4, v);
-    const float inv = inv_norm(ssq, t, eps);
     __builtin_amdgcn_raw_buffer_store_b128(v, xres, lane * 16 + t * (kDim * 4), 0, 0);
+    if (!NORM) continue;
+    const float inv = inv_norm(ssq, t, eps);
     const u32x2 y = {pk_bf16(x[0] * inv, x[1] * inv), pk_bf16(x[2] * inv, x[3] * inv)};
     __builtin_amdgcn_raw_buffer_store_b64(y, nres, lane * 8 + t * (kDim * 2), 0, 0);
   }
@@ -883,7 +884,7 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_res_norm(const uint
   const int64_t tok0 = int64_t(blockIdx.x) * R;
   const int rows = int(n - tok0 < R ? n - tok0 : R);
   const auto xres = buffer_rsrc(X + tok0 * kDim, rows * kDim * 4);
-  const auto nres = buffer_rsrc(xn + tok0 * kDim, xn ? rows * kDim * 2 : 0);
+  const auto nres = buffer_rsrc(xn + tok0 * kDim, rows * kDim * 2);  // (no store without xn)
   const int KS = K / 16, chunks = K / 8, panels = (K + 511) / 512;
   const auto wres = buffer_rsrc(wq + int64_t(wave) * KS * 64, KS * kTileBytes);
   auto stage = [&](int panel) __attribute__((always_inline)) {
@@ -958,9 +959,12 @@ __global__ __launch_bounds__(64 * kTileWaves, 4) void k_gemm_res_norm(const uint
         for (int r = 0; r < 4; ++r) acc[ct][4 * g + r] += b[r];
     }
   }
-  put_ssq(acc, ssq, wave, j, hh);
+  if (xn) put_ssq(acc, ssq, wave, j, hh);
   lds_barrier();
-  store_tile(acc, smem, ssq, eps, xres, nres, wave, lane);
+  if (xn)
+    store_tile<C, true>(acc, smem, ssq, eps, xres, nres, wave, lane);
+  else
+    store_tile<C, false>(acc, smem, ssq, eps, xres, nres, wave, lane);
 }
 
 void launch_gemm_res_norm(const uint16_t* A, int K, const uint8_t* w_packed, const float* bias, float* X,
@@ -1133,7 +1137,7 @@ void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* 
 // The feed-forward runs in bf16, fp16 or split-bf16 operands (PREC, FfPrecision); the out-projection stays
 // bf16.  Split: both FF GEMMs take v = hi + lo (hi = bf16(v), lo = bf16(v - hi)) and form
 // hi.hi + hi.lo + lo.hi with fp32 accumulation; the dropped lo.lo term is ~2^-16 relative.
-// Without OUTPROJ the block starts at X (the feed-forward sub-layer alone); xn may be null (not written).
+// Without OUTPROJ the block starts at X and writes no xn (the feed-forward sub-layer alone).
 //
 // What it replaced: 256-token workgroups whose waves each held all 256 features of 32 tokens and took the
 // weights from LDS in 41 barrier-separated stages (fp16, bf16), and the same with 16 tokens a wave on
@@ -1189,7 +1193,7 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
   const int64_t tok0 = int64_t(blockIdx.x) * R;
   const int rows = int(n - tok0 < R ? n - tok0 : R);  // rows past the last token read as zeros, stores drop
   const auto xres = buffer_rsrc(X + tok0 * kDim, rows * kDim * 4);
-  const auto nres = buffer_rsrc(xn + tok0 * kDim, xn ? rows * kDim * 2 : 0);
+  const auto nres = buffer_rsrc(xn + tok0 * kDim, rows * kDim * 2);  // (no store without OUTPROJ)
   const TileWeights w{buffer_rsrc(layer, int(kLayerBytes)), lane * 16};
   {
     static_assert(kDim * 4 == 512 * 2, "rows of O and X are 1 KB");
@@ -1310,9 +1314,9 @@ __global__ __launch_bounds__(64 * kTileWaves, pa_waves_per_simd(C, PREC)) void k
     put_h();
   }
   tile_gemm<16, C, PREC, 0>(w, ff2(kBlocks - 1).v, out.v, a, acc, hop, none);
-  put_ssq(acc, ssq, wave, j, hh);
+  if (OUTPROJ) put_ssq(acc, ssq, wave, j, hh);
   lds_barrier();
-  store_tile(acc, smem, ssq, eps, xres, nres, wave, lane);
+  store_tile<C, OUTPROJ>(acc, smem, ssq, eps, xres, nres, wave, lane);
 }
 
 namespace {
@@ -1334,8 +1338,8 @@ void launch_post_attn(const uint16_t* O, const uint8_t* layer, float* X, uint16_
   launch_block<true>(O, layer, X, xn, n, ff_precision, eps, st, ev);
 }
 
-void launch_ff(const uint8_t* layer, float* X, uint16_t* xn, int64_t n, int ff_precision, float eps, hipStream_t st) {
-  launch_block<false>(nullptr, layer, X, xn, n, ff_precision, eps, st, LaunchEvents{});
+void launch_ff(const uint8_t* layer, float* X, int64_t n, int ff_precision, float eps, hipStream_t st) {
+  launch_block<false>(nullptr, layer, X, nullptr, n, ff_precision, eps, st, LaunchEvents{});
 }
 
 }  // namespace trf
