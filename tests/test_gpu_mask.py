@@ -1,14 +1,16 @@
 """Mask head on the GPU (trf_mask_head through HipMaskHead) against the oracle.
 
-* tiny model (29 bands of width 16..260, hidden 512), frame counts 1, 31, 33 and 200 (partial 32-frame
-  columns and 128-frame workgroups): ``split`` against the fp64 oracle (final norm + mask estimator,
+* tiny model (29 bands of width 16..260, hidden 512), frame counts 1, 31, 33 and 200 (the kernel for few
+  frames, partial 32-frame workgroups) and 705 and 769 (the 128-frame kernel, partial workgroups and waves; the
+  260 band is jobs of 5 and 4 output pairs): ``split`` against the fp64 oracle (final norm + mask estimator,
   model.py:158-178) at >= 100 dB, the reference's own fp32 parity bar (tests/test_parity.py:25);
   ``fp16`` against the fp64 oracle at >= 60 dB and against the emulation of its rounding points
   (oracle.kernels.mask_head) at >= 85 dB;
 * the reference's golden mask (tests/golden/tiny_forward.npz, written by the reference's
   ``FastBSRoformer._mask``): oracle stack on the CPU, then the HIP mask head, at 100 dB;
-* the full-size model (62 bands of width 8..516, hidden 1024; the 516 and 512 bands are split over
-  three jobs each) at 150 frames against the fp64 oracle, and one full 17 s chunk (1701 frames): a frame's
+* the full-size model (62 bands of width 8..516, hidden 1024) at 150 frames (few: the 512 and 516 bands are
+  four and five jobs) against the fp64 oracle, at 300 in fp16 (the 128-frame kernel: three jobs of 5 and 6 pairs
+  each) band by band against the emulation, and one full 17 s chunk (1701 frames): a frame's
   mask depends on that frame only, so rows of the full launch are checked against the oracle on those
   frames, and two batched chunks give the same rows as one;
 * the output is deterministic, and n_frames = 0 writes nothing.
@@ -45,7 +47,7 @@ def tiny_heads(hip, tiny_sd):
     return {p: HipMaskHead(tiny_sd, TINY, "cuda", precision=p) for p in ("split", "fp16")}
 
 
-@pytest.mark.parametrize("n_frames", [1, 31, 33, 200])
+@pytest.mark.parametrize("n_frames", [1, 31, 33, 200, 705, 769])
 def test_tiny_mask_matches_oracle(tiny_heads, tiny_sd, n_frames):
     dims = weights.band_dims(TINY)
     x = _x(n_frames, len(dims), seed=n_frames)
@@ -99,6 +101,24 @@ def test_full_model_mask_matches_oracle(full_head, full_sd):
     lo = 0
     for f, d in enumerate(dims):  # every band (and every job of the split bands) on its own
         assert snr_db(ref[:, lo : lo + d], got[:, lo : lo + d]) >= 95.0, f"band {f}"
+        lo += d
+
+
+def test_full_model_mask_fp16_matches_its_emulation(hip, full_sd):
+    """Floors as for the tiny model: 60 dB against fp64, 85 against the emulation (80 for a band of 8 columns)."""
+    dims = weights.band_dims(FULL)
+    x = _x(300, len(dims), seed=8)
+    print("full-size mask head, 300 frames, fp16", flush=True)
+    got = HipMaskHead(full_sd, FULL, "cuda", precision="fp16")(x.reshape(-1, 256).cuda()).cpu().numpy()
+    emu = kernels.mask_head(x[0], full_sd, dims, precision="fp16").numpy()
+    ref = _oracle(x, full_sd, FULL).numpy()
+    print(f"  vs fp64 {snr_db(ref, got):.1f} dB, vs its emulation {snr_db(emu, got):.1f} dB")
+    assert snr_db(ref, got) >= 60.0
+    assert snr_db(emu, got) >= 85.0
+    lo = 0
+    for f, d in enumerate(dims):
+        s = snr_db(emu[:, lo : lo + d], got[:, lo : lo + d])
+        assert s >= 80.0, f"band {f}: {s:.1f} dB"
         lo += d
 
 

@@ -4,7 +4,7 @@ of the reference's two ops (qkv_rope_gemm, then attention: kernels.cpp:439-540, 
 library's unfused pair on the same inputs.
 
 Shapes: the 62-band frequency attention (batched, up to the 300-frame chunk), 64 and 33 positions, one
-position, and time attention of chunks of at most 64 frames.  The q and k rows of the weights are scaled up so
+position, time attention of chunks of at most 64 frames, and more sequences than one round of workgroups.  The q and k rows of the weights are scaled up so
 that the scores span tens of units (peaked softmax rows).  Tolerance: the per-op bar of the unfused
 kernels (two bf16 steps elementwise, one rounding flip in 1e-4 of the elements, SNR floor), and every
 output token written.
@@ -34,10 +34,13 @@ SHAPES = [  # (mode, batch, T, F)
     (0, 1, 64, 3),
     (0, 1, 40, 5),
     (0, 2, 1, 5),
-    # group and head splits between the kernel's workgroups (one per CU, an even share of
-    # (4-sequence group, head) units each): 3 x 257 = 771 sequences (1,544 units), 2 x 129 = 258 (520)
+    # more sequences than the workgroups of one launch (256 CUs: 256 of more than 32 positions, 512 of at
+    # most 32), so that they go on to a second and a third one: 771 and 258; 513 and 1,100
     (1, 3, 257, 64),
     (1, 2, 129, 45),
+    (1, 1, 513, 32),
+    (1, 4, 275, 29),
+    (0, 1, 20, 1100),
 ]
 
 
