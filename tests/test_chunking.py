@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from turbo_roformer_amd.chunking import chunk_starts, hamming, overlap_add, step_for
+from turbo_roformer_amd.chunking import chunk_starts, hamming, overlap_add, overlap_add_device, step_for
 from turbo_roformer_amd.separator import as_stereo
 
 
@@ -127,3 +127,11 @@ def test_as_stereo():
                 np.zeros((3, 4), np.float32), np.zeros((2, 2, 2), np.float32)):
         with pytest.raises(ValueError):
             as_stereo(bad)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the error of a machine without a GPU")
+def test_overlap_add_device_without_a_gpu():
+    from turbo_roformer_amd import _hip
+
+    with pytest.raises(_hip.HipUnavailable, match="GPU"):
+        overlap_add_device(torch.zeros(2, 100), 50, 2.0, lambda x: x)

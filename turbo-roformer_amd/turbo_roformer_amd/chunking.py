@@ -114,6 +114,7 @@ def overlap_add_device(
         y = run(torch.stack([x[:, s : s + C] for s in group]).contiguous()).float().contiguous()
         L = min(C, y.shape[-1])
         if w is None:  # formed on the host while the device runs the first chunks
+            _hip.load()  # without a GPU its error, not the one of pinning memory
             w = torch.from_numpy(hamming(C)).pin_memory().to(dev, non_blocking=True)
         _hip.overlap_add(y, L, group, w, acc, wsum)
         if progress is not None:
