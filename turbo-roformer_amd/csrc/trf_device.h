@@ -1,4 +1,4 @@
-// Device helpers shared by the kernel translation units (trf_kernels.hip, trf_mask.hip): operand
+// Device helpers shared by the kernel translation units: operand
 // vector types, the MFMA wrappers, fp16/bf16 packing and the direct-to-LDS weight streaming.
 #pragma once
 

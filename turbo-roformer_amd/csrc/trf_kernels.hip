@@ -148,7 +148,8 @@ void launch_add_rmsnorm(float* X, const void* Y, int y_bf16, void* out, int out_
 // Workgroups of 256 rows that streamed the weights through LDS in 13 barrier-separated stages and stored
 // 8 bytes a lane took 22.6 us at 101 frames x 62 bands (31 workgroups' rows on 256 CUs), 49 at 487 frames and
 // 134 at 1701; these take 15, 34 and 129.  What is left at 1701 is the L2's: a tile's weights pass once per 64
-// positions (the CUs' address units are 70% busy, waiting on it half of that time).
+// positions (the CUs' address units are 70% busy, waiting on it half of that time).  Staging the xn rows costs 4-way
+// bank conflicts, 8% of the cycles.
 // (kernels.cpp:439-540)
 template <int C>
 __global__ __launch_bounds__(64 * kTileWaves, 4) void k_qkv_rope(
@@ -710,7 +711,9 @@ void launch_attention(const uint16_t* Q, const uint16_t* K, const uint16_t* Vt, 
     // Two column tiles a wave share each operand read of a 256-query workgroup; one makes a 128-query
     // workgroup, for an odd number of 128-query blocks, whose last 256-query one would run half empty. us at
     // 62 bands, QT = 2 and 1: L = 101 11.2 and 9.6, 257 30.8 and 24.2, 384 35.3 and 30.3, 520 58.3 and 55.9,
-    // 640 65.3 and 64.5, 896 114 and 114 (even numbers of blocks: 200 18.6 and 19.2, 800 102 and 101).
+    // 640 65.3 and 64.5, 896 114 and 114 (even numbers of blocks: 200 18.6 and 19.2, 800 102 and 101). With few and
+    // with many sequences alike: L = 257 10.3 and 9.1 at 4, 216 and 173 at 496; 640 15.0 and 10.5 at 4, 213 and 192
+    // at 186.
     const int blocks = (sh.L + att_block_q(1) - 1) / att_block_q(1);
     const int QT = blocks % 2 && blocks <= 5 ? 1 : 2;
     const int nqb = (sh.L + att_block_q(QT) - 1) / att_block_q(QT);
@@ -1145,7 +1148,9 @@ void launch_gemm_gelu(const uint16_t* xn, const uint8_t* w_packed, const float* 
 // 80 and 21.5 at 6,262; the feed-forward alone 74 and 38 at 18,786 (fp16), 365 and 319 at 105,462 (split).
 // At 105,462 tokens the parts are 74 us of HBM traffic (378 MB at the rate of a copy), 56 us of MFMA work
 // and, without either, ~30 us for the weights' way from L2; the tiles of a round start together, so they
-// overlap only in part (priorities for one of a CU's two workgroups change nothing).
+// overlap only in part (priorities for one of a CU's two workgroups change nothing). In cycles the fp16 block is 22%
+// shorter there, 446k and 348k; the chip's power limit takes the clock from 2.27 to 1.95 GHz, also under the kernels
+// beside it. The split block at C = 1 keeps 4 registers in scratch.
 // (fast.py:311-331, kernels.cpp:542-642)
 
 // FF operand packing of the one-part arithmetics.

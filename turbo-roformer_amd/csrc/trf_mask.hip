@@ -71,9 +71,10 @@ struct MaskOps {
 // One stage.  pre holds tile u-1's pre-activations.  LAST: tanh and GEMM2 of the last hidden tile only.
 // Otherwise: tanh(pre) into the GEMM2 B operands, one value after each GEMM1 unit, then GEMM2(u-1) with
 // the sums of tile u's pre-activations (the two chains and b1) between its MFMAs: at the start of the next
-// stage they would stand alone, 64 instructions of the wave's single SIMD.  dma(q) issues this wave's q-th direct-to-LDS block of the next stage
-// after unit q.  (Issued all at once, the next stage's 40-80 KB per workgroup outrun what a CU keeps in
-// flight and the wave stalls in issue before its MFMAs; spread over the first units, they stream under
+// stage they would stand alone, 64 instructions of the wave's single SIMD (17 s chunk, split: 284 -> 279 us on
+// a repeated input, 312 -> 307 on one that has to come from HBM).  dma(q) issues this wave's q-th direct-to-LDS
+// block of the next stage after unit q.  (Issued all at once, the next stage's 40-80 KB per workgroup outrun what a
+// CU keeps in flight and the wave stalls in issue before its MFMAs; spread over the first units, they stream under
 // them and land before the stage ends.)  Each unit's operand blocks are read one unit ahead.
 template <bool SPLIT, int NP, bool LAST, typename Dma>
 __device__ __forceinline__ void mask_stage(const u32x4* L, int u, const float* b1, const u32x4 (&xh)[16],

@@ -25,9 +25,10 @@
 // O leaves through the wave's own LDS rows as whole 128-byte lines.
 //
 // Against workgroups of 4 sequences that streamed the weights through LDS and exchanged K and V^T between
-// position halves (us): 62 positions, 251 sequences 35 and 23; 101 sequences 19.5 and 17; 1701 the same within 1%.  At 1701 the
-// MFMA pipe is busy 40%, the address units 46%, LDS 36% of the time; 8 weight k-steps ahead instead of 4, and
-// 8 heads a workgroup instead of 4, changed nothing there.
+// position halves (us): 62 positions, 251 sequences 35 and 23; 101 sequences 19.5 and 17; 1701 the same within 3%
+// (264k cycles and 250k, at a lower clock).  At 1701 the MFMA pipe is busy 39%, the address units 50%, LDS 35% of the
+// time, 11% of the cycles go to the bank conflicts of staging xn, and C = 2 keeps 12 registers in scratch; 8 weight
+// k-steps ahead instead of 4, and 8 heads a workgroup instead of 4, changed nothing there.
 #include "trf_tiles.h"
 
 namespace trf {

@@ -9,7 +9,11 @@
 // delivers ~50 bytes per cycle per CU, which bounds C = 1 (1.3 MB of weights per 32 tokens in the
 // post-attention block); C = 4 fills a CU with one workgroup.  That block in us at C = 1 / 2 / 4: 18 / 24 /
 // 45 at 6,262 tokens, 37 / 35 / 53 at 16,384, 223 / 172 / 225 at 105,462.  So a launch takes C = 1 while its
-// 32-token tiles fit one per CU and C = 2 beyond.
+// 32-token tiles fit one per CU and C = 2 beyond (the residual GEMM's own rule is at its launch).  Between, us at
+// C = 1 and 2, feed-forward in fp16: 23.1 and 19.8 at 8,246, 36.1 and 36.1 at 16,492, 54 and 44 at 30,194, 61 and 58
+// at 32,984, 101 and 83 at 62,000; in split: 42 and 35 at 8,246, 70 and 77 at 16,492 (C = 2 has one workgroup a CU and
+// starts its second round there), 102 and 90 at 30,194, 201 and 180 at 62,000; time QKV: 20 and 16 at 8,246, 31 and 27
+// at 16,492, 45 and 33 at 30,194, 87 and 62 at 62,000.
 //
 // Rows of activations move in whole rows or half rows per wave instruction and are transposed through LDS.
 // Loaded or stored in operand layout (32 rows x 16 bytes, the halves of a pair 32 lanes apart) an
